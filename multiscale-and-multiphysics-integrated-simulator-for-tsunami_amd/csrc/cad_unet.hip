@@ -31,7 +31,8 @@
 // Blocks of neighbouring rows are dealt to the same XCD, so the rows they
 // share stay in one L2.  The backward pass for the activations is the same
 // kernel with the taps flipped and the weight matrix transposed (packed that
-// way), and the weight gradients are an FP32 reduction over voxels.
+// way), and the weight gradients are a product over the voxels on the matrix
+// cores.
 //
 // A convolution's input may come from two buffers (the decoder's skip
 // concatenation: channels below `split` from the upsampled coarse features,
@@ -541,119 +542,178 @@ __global__ void k_pack(const float *__restrict__ w, int cin, int cout, int flip,
     }
 }
 
-// FP32 weight gradient of one 3x3x3 layer: dW[t][ci][co] += sum_v X[v+off_t][ci] dY[v][co]
-// and (tap 13's blocks) db[co] += sum_v dY[v][co].  Block: one tap, a range of
-// interior voxels; threads own 4x4 (ci, co) blocks, several thread groups
-// split each tile of voxels; partial sums are added atomically.
+// Weight gradient of one 3x3x3 layer on the matrix cores: dW[t][ci][co] =
+// sum_v X[v+off_t][ci] dY[v][co] and db[co] = sum_v dY[v][co], a product whose
+// long dimension is the voxels.  BF16 inputs, exact products, FP32 sums, as
+// the forward convolution.
+//
+// blockIdx.y is the z tap.  A block takes units (a run of yr rows of one z
+// plane and one 64-voxel x segment) blockIdx.x, + gridDim.x, ... and marches
+// their rows: the X rows y-1 .. y+1 (with one halo voxel on each side) and dY's
+// row y sit in LDS as they come, channels last, the next ones in flight in
+// registers.  The nine (y, x) taps are then address offsets, so an X row is
+// read from HBM once per z tap, and both fragments come out of LDS transposed
+// (ds_read_b64_tr_b16: four voxels of one channel per lane).  The record
+// pitches put the eight records that a read touches in eight different bank
+// groups.  The wave owns the (tap, 16 input channels) rows wave, wave + 4, ...
+// for all output channels, so a dY fragment serves all of them.
+//
+// Blocks store their partial sums and k_dw_sum adds them in block order, so the
+// gradients are the same from run to run.  On a batch of 8 boxes of 64x32x32
+// the twelve layers take 0.34 ms and their sums 0.14 ms, where one-tap blocks on
+// the vector units with atomic sums took 14.4 ms (54 GFLOP: 3.8 -> 110
+// TFLOP/s).  Bound by the LDS reads of the fragments and, at 16 channels, by
+// the march's one barrier a row.
+constexpr int DW_SEG = 64;                       // voxels of an x segment
+constexpr int DW_PART_BYTES = 32 << 20;          // partial sums of a layer at most
+__host__ __device__ constexpr int dw_pitch(int c) { return c <= 16 ? c : c + 16; }   // bf16 per LDS record
+
 template <int CIN, int COUT>
-__global__ void __launch_bounds__(256) k_conv_dw(UGeo g, ConvIn x,
-                                                 const bf16 *__restrict__ dy, int cs_dy,
-                                                 long long per_block, float *__restrict__ dw,
-                                                 float *__restrict__ db)
+__global__ void __launch_bounds__(256) k_conv_dw(UGeo g, ConvIn x, const bf16 *__restrict__ dy, int cs_dy,
+                                                 int nseg, int yr, int units, float *__restrict__ part)
 {
-    constexpr int TV = 32;
-    constexpr int NBLK = (CIN / 4) * (COUT / 4);
-    constexpr int GROUPS = NBLK >= 256 ? 1 : 256 / NBLK;
-    __shared__ float xs[TV][CIN + 1];
-    __shared__ float ds[TV][COUT + 1];
-    __shared__ float red[GROUPS > 1 ? GROUPS : 1][NBLK > 256 ? 1 : NBLK][17];
-    const int t = blockIdx.y;
-    const long long off = tap_off(g, t);
-    const long long total = (long long)g.nx * g.ny * g.nz * g.nb;
-    const long long u0 = blockIdx.x * per_block;
-    const long long u1 = u0 + per_block < total ? u0 + per_block : total;
-    const int tid = threadIdx.x;
-    // thread -> (group, 4x4 block)
-    const int grp = tid / (NBLK >= 256 ? 256 : NBLK);
-    const int blk0 = tid % (NBLK >= 256 ? 256 : NBLK);
-    constexpr int BPT = NBLK > 256 ? NBLK / 256 : 1;   // 4x4 blocks per thread
-    float acc[BPT][16];
-    float dbacc[BPT][4];
+    constexpr int MT = (CIN + 15) / 16, NT = COUT / 16;
+    constexpr int XP = dw_pitch(CIN), DP = dw_pitch(COUT);
+    constexpr int ROWS = 9 * MT, NA = (ROWS + 3) / 4;
+    constexpr int XC = CIN / 8, DC = COUT / 8;   // 16-byte pieces of a record
+    constexpr int XL = ((DW_SEG + 2) * XC + 255) / 256, DL = (DW_SEG * DC + 255) / 256;
+    typedef short s4 __attribute__((ext_vector_type(4)));
+    typedef __attribute__((address_space(3))) s4 lds_s4;
+    // 8 input channels: a read of 16 takes the next record's, and the last
+    // record's reads end 8 channels past it; those rows of dW are not stored
+    __shared__ bf16x8 xs_[(4 * (DW_SEG + 2) * XP + 16) / 8];
+    __shared__ bf16x8 ds_[2 * DW_SEG * DP / 8];
+    bf16 *xs = reinterpret_cast<bf16 *>(xs_), *ds = reinterpret_cast<bf16 *>(ds_);
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int dz = (int)blockIdx.y - 1;
+    // a lane's part of a transposed read: voxel 4 (l/16) + l%16/4 of the step's
+    // sixteen, channels 4 (l%4) .. +3; it gets channel l%16 of voxels 4 (l/16) .. +3
+    const int fv = 4 * (lane >> 4) + ((lane >> 2) & 3), fc = 4 * (lane & 3);
+    f4 acc[NA][NT], bacc[NT];
 #pragma unroll
-    for (int p = 0; p < BPT; p++) {
+    for (int q = 0; q < NA; q++)
 #pragma unroll
-        for (int e = 0; e < 16; e++) acc[p][e] = 0.f;
+        for (int n = 0; n < NT; n++) acc[q][n] = f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int e = 0; e < 4; e++) dbacc[p][e] = 0.f;
-    }
-    for (long long ub = u0; ub < u1; ub += TV) {
-        __syncthreads();
-        for (int e = tid; e < TV * (CIN + COUT); e += 256) {
-            const int vi = e / (CIN + COUT), c = e % (CIN + COUT);
-            const long long u = ub + vi;
-            float val = 0.f;
-            if (u < u1) {
-                const long long v = vox_of(g, u);
-                val = c < CIN ? (float)*chan(x, v + off, c) : (float)dy[v * cs_dy + (c - CIN)];
+    for (int n = 0; n < NT; n++) bacc[n] = f4{0.f, 0.f, 0.f, 0.f};
+    const s4 ones = {0x3F80, 0x3F80, 0x3F80, 0x3F80};   // BF16 1.0
+    const bool bias = dz == 0 && wave == 3;
+    const int runs = (g.ny + yr - 1) / yr;
+
+    for (int u = blockIdx.x; u < units; u += gridDim.x) {
+        const int sx = u % nseg, yq = u / nseg % runs, zb = u / nseg / runs;
+        const int z = zb % g.nz, b = zb / g.nz;
+        const int x0 = sx * DW_SEG, len = min(DW_SEG, g.nx - x0);
+        const int y0 = yq * yr, y1 = min(y0 + yr, g.ny);
+        bf16x8 xr[XL], dr[DL];
+        auto fetch_x = [&](int y) {
+            const long long v0 = vox(g, x0 - 1, y, z + dz, b);
+#pragma unroll
+            for (int e = 0; e < XL; e++) {
+                const int i = tid + 256 * e;
+                if (i < (len + 2) * XC) xr[e] = *reinterpret_cast<const bf16x8 *>(chan(x, v0 + i / XC, 8 * (i % XC)));
             }
-            if (c < CIN)
-                xs[vi][c] = val;
-            else
-                ds[vi][c - CIN] = val;
+        };
+        auto fetch_d = [&](int y) {
+            const long long v0 = vox(g, x0, y, z, b);
+#pragma unroll
+            for (int e = 0; e < DL; e++) {
+                const int i = tid + 256 * e;
+                if (i < len * DC) dr[e] = *reinterpret_cast<const bf16x8 *>(dy + (v0 + i / DC) * cs_dy + 8 * (i % DC));
+            }
+        };
+        auto put_x = [&](int y) {
+            bf16 *row = xs + (y & 3) * (DW_SEG + 2) * XP;
+#pragma unroll
+            for (int e = 0; e < XL; e++) {
+                const int i = tid + 256 * e;
+                if (i < (len + 2) * XC) *reinterpret_cast<bf16x8 *>(row + (i / XC) * XP + 8 * (i % XC)) = xr[e];
+            }
+        };
+        auto put_d = [&](int y) {
+            bf16 *row = ds + (y & 1) * DW_SEG * DP;
+#pragma unroll
+            for (int e = 0; e < DL; e++) {
+                const int i = tid + 256 * e;
+                if (i < len * DC) *reinterpret_cast<bf16x8 *>(row + (i / DC) * DP + 8 * (i % DC)) = dr[e];
+            }
+        };
+        __syncthreads();   // the last unit's rows are read
+        for (int y = y0 - 1; y <= y0 + 1; y++) {
+            fetch_x(y);
+            put_x(y);
         }
+        fetch_d(y0);
+        put_d(y0);
         __syncthreads();
-        if (grp < GROUPS) {
+        for (int y = y0; y < y1; y++) {
+            if (y + 1 < y1) {
+                fetch_x(y + 2);
+                fetch_d(y + 1);
+            }
+            const bf16 *drow = ds + (y & 1) * DW_SEG * DP + fv * DP + fc;
+            const bf16 *arow[NA];
 #pragma unroll
-            for (int p = 0; p < BPT; p++) {
-                const int blk = blk0 + p * 256;
-                const int bi = blk / (COUT / 4), bo = blk % (COUT / 4);
-                for (int vi = grp; vi < TV; vi += GROUPS) {
-                    float xv[4], dv[4];
+            for (int q = 0; q < NA; q++) {
+                const int a = min(wave + 4 * q, ROWS - 1);
+                const int t = a / MT, m = a % MT;
+                arow[q] = xs + (((y + t / 3 - 1) & 3) * (DW_SEG + 2) + t % 3 + fv) * XP + 16 * m + fc;
+            }
+            for (int k = 0; k < len; k += 16) {
+                s4 bf[NT];
 #pragma unroll
-                    for (int a = 0; a < 4; a++) {
-                        xv[a] = xs[vi][4 * bi + a];
-                        dv[a] = ds[vi][4 * bo + a];
-                    }
+                for (int n = 0; n < NT; n++)
+                    bf[n] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4 *)(drow + k * DP + 16 * n));
 #pragma unroll
-                    for (int a = 0; a < 4; a++)
+                for (int q = 0; q < NA; q++) {
+                    if (wave + 4 * q >= ROWS) continue;
+                    const s4 af = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4 *)(arow[q] + k * XP));
 #pragma unroll
-                        for (int c = 0; c < 4; c++) acc[p][a * 4 + c] += xv[a] * dv[c];
-                    if (bi == 0)
-#pragma unroll
-                        for (int c = 0; c < 4; c++) dbacc[p][c] += dv[c];
+                    for (int n = 0; n < NT; n++)
+                        acc[q][n] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(af, bf[n], acc[q][n], 0, 0, 0);
                 }
+                if (bias)
+#pragma unroll
+                    for (int n = 0; n < NT; n++)
+                        bacc[n] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(ones, bf[n], bacc[n], 0, 0, 0);
             }
+            if (y + 1 < y1) {
+                put_x(y + 2);
+                put_d(y + 1);
+            }
+            __syncthreads();
         }
     }
-    // reduce over the thread groups, then one atomic per weight
-    if (GROUPS > 1) {
-        __syncthreads();
-        if (grp < GROUPS) {
+    // D of the product: row (ci) 4 (l/16) + r, column (co) l%16
+    float *p = part + (long long)blockIdx.x * (27 * CIN * COUT + COUT);
 #pragma unroll
-            for (int e = 0; e < 16; e++) red[grp][blk0][e] = acc[0][e];
-        }
-        __syncthreads();
-        if (grp == 0) {
-            for (int gq = 1; gq < GROUPS; gq++)
+    for (int q = 0; q < NA; q++) {
+        const int a = wave + 4 * q;
+        if (a >= ROWS) continue;
+        const int t = 9 * (int)blockIdx.y + a / MT, c0 = 16 * (a % MT) + 4 * (lane >> 4);
 #pragma unroll
-                for (int e = 0; e < 16; e++) acc[0][e] += red[gq][blk0][e];
-        }
-        __syncthreads();
-        if (grp < GROUPS) {
+        for (int n = 0; n < NT; n++)
 #pragma unroll
-            for (int e = 0; e < 4; e++) red[grp][blk0][e] = dbacc[0][e];
-        }
-        __syncthreads();
-        if (grp == 0) {
-            for (int gq = 1; gq < GROUPS; gq++)
-#pragma unroll
-                for (int e = 0; e < 4; e++) dbacc[0][e] += red[gq][blk0][e];
-        }
+            for (int r = 0; r < 4; r++)
+                if (c0 + r < CIN) p[((long long)t * CIN + c0 + r) * COUT + 16 * n + (lane & 15)] = acc[q][n][r];
     }
-    if (grp != 0) return;
+    if (bias && lane < 16)
 #pragma unroll
-    for (int p = 0; p < BPT; p++) {
-        const int blk = blk0 + p * 256;
-        const int bi = blk / (COUT / 4), bo = blk % (COUT / 4);
-#pragma unroll
-        for (int a = 0; a < 4; a++)
-#pragma unroll
-            for (int c = 0; c < 4; c++)
-                atomicAdd(&dw[((long long)t * CIN + 4 * bi + a) * COUT + 4 * bo + c], acc[p][a * 4 + c]);
-        if (t == 13 && bi == 0 && db)
-#pragma unroll
-            for (int c = 0; c < 4; c++) atomicAdd(&db[4 * bo + c], dbacc[p][c]);
-    }
+        for (int n = 0; n < NT; n++) p[27 * CIN * COUT + 16 * n + lane] = bacc[n][0];
+}
+
+// a layer's weight and bias gradients (adjacent in the parameter vector) from
+// the blocks' partial sums, in block order
+__global__ void __launch_bounds__(256) k_dw_sum(int n, int blocks, const float *__restrict__ part,
+                                                float *__restrict__ dw)
+{
+    const int e = blockIdx.x * 256 + threadIdx.x;
+    if (e >= n) return;
+    float s = 0.f;
+#pragma unroll 8
+    for (int b = 0; b < blocks; b++) s += part[(long long)b * n + e];
+    dw[e] += s;
 }
 
 // Element-wise kernels run over the x rows of a level: block b covers
@@ -906,6 +966,7 @@ struct cad_unet {
     bf16 *dh1e, *dh1d, *dcat1a, *dcat1b, *dh2f, *dh2e, *dh2d, *dcat2a, *dcat2b, *dh3c, *dh3b, *dh3a, *dp2, *dh2a,
         *dp1, *dh1a;
     float *y, *dy, *esq, *loss;
+    float *dwpart;                  // blocks' partial sums of a layer's weight gradient
     bool train;
     long long step;
     std::vector<void *> allocs;
@@ -1090,16 +1151,26 @@ int layer_bwd(cad_unet *u, int l, const ConvIn &in, const bf16 *dy, int cs_dy, c
         int rc = conv(u, g, L.cout, one_in(dy, cs_dy, L.cout), u->wt[l], nullptr, *dx, L.cin, false);
         if (rc) return rc;
     }
-    const long long total = (long long)g.nx * g.ny * g.nz * g.nb;
-    const long long per = 4096;
-    const dim3 grid((unsigned)((total + per - 1) / per), 27), blk(256);
-    float *dw = u->gr + u->wofs[l], *db = u->gr + u->bofs[l];
-#define CAD_DW(CI, CO)                                                                                \
-    if (L.cin == CI && L.cout == CO)                                                                  \
-        hipLaunchKernelGGL((k_conv_dw<CI, CO>), grid, blk, 0, u->stream, g, in, dy, cs_dy, per, dw, db);
+    const int n = 27 * L.cin * L.cout + L.cout;
+    const int nseg = (g.nx + DW_SEG - 1) / DW_SEG;
+    // blocks: as many as fill the chip's CUs (each counts three times, once per z
+    // tap) and as the partial sums have room for; runs of rows are halved
+    // until there are that many units, down to 4 (a run reads two rows more
+    // than it computes)
+    const int want = std::min(u->ncu, (int)(DW_PART_BYTES / (n * sizeof(float))));
+    int yr = g.ny;
+    auto units = [&](int r) { return (long long)nseg * ((g.ny + r - 1) / r) * g.nz * g.nb; };
+    while (yr > 4 && units(yr) < want) yr = std::max(4, (yr + 1) / 2);
+    const int blocks = (int)std::min<long long>(units(yr), want);
+#define CAD_DW(CI, CO)                                                                                    \
+    if (L.cin == CI && L.cout == CO)                                                                      \
+        hipLaunchKernelGGL((k_conv_dw<CI, CO>), dim3(blocks, 3), dim3(256), 0, u->stream, g, in, dy, cs_dy, nseg, \
+                           yr, (int)units(yr), u->dwpart);
     CAD_DW(8, 16) CAD_DW(16, 16) CAD_DW(16, 32) CAD_DW(32, 32) CAD_DW(32, 64) CAD_DW(64, 64)
     CAD_DW(64, 32) CAD_DW(32, 16)
 #undef CAD_DW
+    hipLaunchKernelGGL(k_dw_sum, dim3((n + 255) / 256), dim3(256), 0, u->stream, n, blocks, u->dwpart,
+                       u->gr + u->wofs[l]);
     CAD_CHECK(hipGetLastError());
     return CAD_OK;
 }
@@ -1335,6 +1406,7 @@ int cad_unet_create(int nx, int ny, int nz, int nb, int train, void *stream, cad
         A(&u->dy, nvox(u->g[0]));
         A(&u->esq, (size_t)nb);
         A(&u->loss, 1);
+        A(&u->dwpart, DW_PART_BYTES / sizeof(float));
     }
     if (!rc && hipStreamSynchronize(u->stream) != hipSuccess) rc = CAD_ERR_HIP;
     if (rc) {

@@ -140,3 +140,42 @@ def test_unet_adam_steps_lower_the_loss(pkg):
     print(f"loss {losses[0]:.4f} -> {losses[-1]:.4f}", flush=True)
     assert losses[-1] < 0.8 * losses[0]
     assert np.all(np.isfinite(losses))
+
+
+@pytest.mark.parametrize("box,nb", [((64, 4, 4), 1), ((192, 12, 20), 3), ((320, 36, 4), 1)])
+def test_unet_weight_gradients_by_segments_and_runs(pkg, box, nb):
+    """The weight gradients' blocks at the edges of their split: one row and
+    one 16-voxel segment on the coarsest level, x segments with a remainder
+    (96 = 64 + 32 and 160 = 2 x 64 + 32 voxels on the middle level), row runs
+    with a remainder, fewer and more units than blocks.  The bar is the one
+    above; the partial sums are added in a fixed order, so two calls give the
+    same bits, apart from the output layer's 17 sums and what the loss's
+    atomic sum moves: dy is given, so nothing."""
+    import torch
+    U = pkg.unet
+    nx, ny, nz = box
+    p, pr, xf, xp, e, m = _setup(pkg, box, nb, 7)
+    with U.UNet(nx, ny, nz, nb, train=True) as net:
+        net.set_params(p)
+        net.set_input(xp.cuda())
+        y = torch.empty(nb * nz * ny * nx, dtype=torch.float32, device="cuda")
+        net.forward(y)
+        dy = (2.0 * torch.from_numpy(m).cuda() * (y.view(nb, nz, ny, nx) - torch.from_numpy(e).cuda())).reshape(-1)
+        torch.cuda.synchronize()
+        g = net.gradients_dy(dy)
+        g2 = net.gradients_dy(dy)
+    prm = unet_ref.forward(U, pr, xf)
+    for v in prm.values():
+        v[0].requires_grad_(True)
+        v[1].requires_grad_(True)
+    yr = unet_ref.run(prm, xf)
+    (yr * dy.cpu().view(nb, nz, ny, nx)).sum().backward()
+    gr = unet_ref.grad_vector(U, prm, U.param_count())
+    sl = U.layer_slices()
+    for name in U.NAMES:
+        for part in (0, 1):
+            a, b = g[sl[name][part]], gr[sl[name][part]]
+            rel = np.linalg.norm(a - b) / np.linalg.norm(b)
+            print(f"{name} {'wb'[part]}: rel {rel:.3e}", flush=True)
+            assert rel <= 1e-1, (name, part, rel)
+            assert np.array_equal(a, g2[sl[name][part]]), (name, part)
