@@ -227,6 +227,7 @@ void cad_destroy(cad_ctx *c)
     for (void *p : ptrs)
         if (p) hipFree(p);
     cad_sweep_free(c);
+    cad_wave_sweep_free(c);
     cad_tdoor_free(c);
     cad_wave_free(c);
     cad_wave_theory_free(c);

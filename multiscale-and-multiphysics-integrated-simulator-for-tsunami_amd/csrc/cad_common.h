@@ -179,6 +179,10 @@ struct cad_ctx {
     unsigned long long *sw_ticket;
     unsigned long long sw_base;
     unsigned sw_seq;
+    // packed sweeps (cad_wave_sweep.hip): their arrays, null until the first
+    // plain solve; not to be allocated; the current factorisation is packed
+    struct cad_wsweep *ws;
+    bool ws_off, ws_packed;
     // VOF work: F fluxes
     double *flf[3];
     // scratch for reductions and counters
@@ -318,6 +322,10 @@ int cad_sweep_bind(cad_ctx *c, char *base, unsigned long long bytes, unsigned se
 int cad_sweep_dcmp(cad_ctx *c, double u, int *npos_host);
 int cad_sweep_minv(cad_ctx *c, double *x, const double *y);
 int cad_sweep_status(cad_ctx *c, int *code);
+int cad_wave_alloc(cad_ctx *c);
+void cad_wave_sweep_free(cad_ctx *c);
+int cad_wave_pack(cad_ctx *c);
+int cad_wave_minv(cad_ctx *c, double *x, const double *y);
 int cad_milu_factor_impl(cad_ctx *c, int *npos);
 int cad_poisson_residual_impl(cad_ctx *c, double *rel);
 int cad_poisson_residual_x(cad_ctx *c, const double *x, double *rel);

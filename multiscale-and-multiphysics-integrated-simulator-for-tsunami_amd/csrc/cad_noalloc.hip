@@ -126,6 +126,7 @@ extern "C" int cad_m1bcgs_noalloc(void *stream, const double *ad, const double *
     c.d.nij = (long long)ni * nj;
     c.d.nc = nc;
     c.sweep_schedule = CAD_SWEEP_PIPELINED;
+    c.ws_off = true;   // no allocation: the natural-layout sweeps
     if (cad_sweep_bytes(&c) > SWEEP_BYTES) {
         cad_set_error("cad_m1bcgs_noalloc: the sweeps of %d x %d x %d need %llu bytes of mailboxes, "
                       "more than the %llu reserved", ni, nj, nk, cad_sweep_bytes(&c), SWEEP_BYTES);

@@ -54,6 +54,7 @@
 // INDC: the precomputed LP*/AU* arrays carry a marker value at inactive cells,
 // and DD is zero there and positive at active cells.
 #include "cad_common.h"
+#include "cad_sweep.h"
 
 #include <algorithm>
 #include <climits>
@@ -61,48 +62,7 @@
 
 namespace {
 
-constexpr unsigned SPIN_LIMIT = 1u << 20;
-constexpr unsigned OOB = 0xFFFFFFF0u;
-constexpr int CPOL_DEVICE = 16;      // sc1: device-scope coherent access
 constexpr int MB_LINES = 16;         // mailbox lines per tile and side (max of TJ, TK)
-// inactive-cell marker: a signalling-NaN pattern that no arithmetic produces
-constexpr unsigned long long MARK = 0x7FF4DEADBEEF0001ull;
-
-typedef unsigned v4u __attribute__((ext_vector_type(4)));
-typedef unsigned v3u __attribute__((ext_vector_type(3)));
-typedef unsigned v2u __attribute__((ext_vector_type(2)));
-typedef __attribute__((address_space(3))) void lds_void;
-
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(const void *p, unsigned long long bytes)
-{
-    const unsigned nrec = bytes > 0xFFFFFFF0ull ? 0xFFFFFFF0u : (unsigned)bytes;
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, (int)nrec, 0x00020000);
-}
-
-// 16 bytes per lane from buffer offset off straight into LDS at lds + 16*lane
-__device__ __forceinline__ void load_lds16(__amdgpu_buffer_rsrc_t r, void *lds, unsigned off)
-{
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void *)lds, 16, off, 0, 0, 0);
-}
-
-__device__ __forceinline__ bool is_mark(double x)
-{
-    return __builtin_bit_cast(unsigned long long, x) == MARK;
-}
-
-// {value, sequence number} of a mailbox entry: 12 bytes inside the 16-byte
-// entry that one store wrote
-__device__ __forceinline__ v3u mb_load(__amdgpu_buffer_rsrc_t r, unsigned off)
-{
-    return __builtin_amdgcn_raw_buffer_load_b96(r, off, 0, CPOL_DEVICE);
-}
-
-__device__ __forceinline__ void mb_store(__amdgpu_buffer_rsrc_t r, unsigned off, double x, unsigned seq)
-{
-    const v2u b = __builtin_bit_cast(v2u, x);
-    const v4u e = {b.x, b.y, seq, seq};
-    __builtin_amdgcn_raw_buffer_store_b128(e, r, off, 0, CPOL_DEVICE);
-}
 
 // Slow path of a mailbox read: polls the entry until it carries sequence
 // number seq, at most SPIN_LIMIT times (then flags err and returns what it
@@ -878,6 +838,12 @@ void cad_sweep_free(cad_ctx *c)
 int cad_sweep_dcmp(cad_ctx *c, double u, int *npos_host)
 {
     const Dims &d = c->d;
+    // the default schedule packs the factorisation for the sweeps of
+    // cad_wave_sweep.hip where their arrays fit
+    const bool pack = c->sweep_schedule == CAD_SWEEP_PIPELINED;
+    if (pack)
+        if (int rc = cad_wave_alloc(c)) return rc;
+    c->ws_packed = pack && c->ws;
     hipLaunchKernelGGL(k_set_int, dim3(1), dim3(1), 0, c->stream, c->icount + 3, -1);
     for (int sh = 0; sh < 2; sh++) {
         SweepGeom g = geom(c, sh);
@@ -925,9 +891,13 @@ int cad_sweep_dcmp(cad_ctx *c, double u, int *npos_host)
     op.out = c->dd;
     op.flag = c->icount + 1;
     if (int rc = launch<DcmpOp, 1>(c, op)) return rc;
-    hipLaunchKernelGGL(k_lprod, cell_grid(d), cell_block(), 0, c->stream, d, c->ali, c->alj,
-                       c->alk, c->dd, c->f.indc, c->lpi, c->lpj, c->lpk);
-    CAD_CHECK(hipGetLastError());
+    if (c->ws_packed) {
+        if (int rc = cad_wave_pack(c)) return rc;
+    } else {
+        hipLaunchKernelGGL(k_lprod, cell_grid(d), cell_block(), 0, c->stream, d, c->ali, c->alj,
+                           c->alk, c->dd, c->f.indc, c->lpi, c->lpj, c->lpk);
+        CAD_CHECK(hipGetLastError());
+    }
     CAD_CHECK(hipMemcpyAsync(c->host_cnt + 1, c->icount + 1, sizeof(int), hipMemcpyDeviceToHost, c->stream));
     CAD_CHECK(hipMemcpyAsync(c->host_cnt + 2, c->sw_err, sizeof(int), hipMemcpyDeviceToHost, c->stream));
     CAD_CHECK(hipStreamSynchronize(c->stream));
@@ -942,6 +912,7 @@ int cad_sweep_dcmp(cad_ctx *c, double u, int *npos_host)
 // x = M^-1 y (vf_mzminv.f:38-41): forward then backward sweep, in place on x.
 int cad_sweep_minv(cad_ctx *c, double *x, const double *y)
 {
+    if (c->ws_packed) return cad_wave_minv(c, x, y);
     FwdOp f;
     f.src[0] = y;
     f.src[1] = c->lpi;

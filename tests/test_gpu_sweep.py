@@ -158,3 +158,39 @@ def test_milu_apply_bitexact_many_tiles(pkg, sched):
     prm = {k: v for k, v in p.items() if k in ("cgpara", "icgtyp", "cgepsa", "cgepsr", "cgdiv", "icgmax")}
     rs = np.random.default_rng(11)
     _milu_check(pkg, mat, indc, prm, sched, [mat["BB"], rs.standard_normal(mat["AD"].shape)])
+
+
+@pytest.mark.parametrize("shape", [(4, 3, 3), (9, 16, 4), (14, 17, 9), (21, 2, 40), (37, 49, 5), (600, 11, 6),
+                                   (301, 21, 13)])
+def test_packed_sweeps_bitexact_with_oracle(pkg, shape):
+    """The default schedule's packed sweeps at the edges of their tiles (16 x 4
+    and 16 x 8 lines, stages of 8 steps, one and two walking waves a
+    workgroup), on matrices with random couplings and activity: whole lines
+    and tiles without an active cell, activity that ends anywhere in a stage,
+    values on inactive cells of the right-hand side and the matrix that must
+    not be read.  M^-1 y equals the oracle's serial sweeps bit for bit, twice in
+    a row (the second call's mailboxes hold the first one's entries)."""
+    ni, nj, nk = (n + 2 for n in shape)
+    rs = np.random.default_rng(ni * 131 + nj)
+    indc = np.full((ni, nj, nk), -1, np.int32, order="F")
+    act = rs.random(shape) < 0.8
+    act[:, rs.random(shape[1]) < 0.2, :] = False
+    act[:, :, shape[2] * 3 // 4 + 1:] = False
+    act[: shape[0] // 5] = False
+    act[shape[0] // 2, shape[1] // 2, 0] = True
+    indc[1:-1, 1:-1, 1:-1] = np.where(act, 0, -1)
+    on = indc == 0
+    mat = {k: np.zeros((ni, nj, nk), order="F") for k in pkg.capi.MATRIX}
+    for a, (lo, up) in enumerate((("ALI", "AUI"), ("ALJ", "AUJ"), ("ALK", "AUK"))):
+        w = -rs.random((ni, nj, nk))
+        back = np.roll(on, 1, axis=a)
+        mat[lo][...] = np.where(on & back, w, 0.0)
+        mat[up][...] = np.roll(mat[lo], -1, axis=a)
+    mat["AD"][...] = 6.5
+    mat["BB"][...] = rs.standard_normal((ni, nj, nk))
+    for k in ("AUI", "ALJ", "AD"):      # never read on inactive cells
+        mat[k][1:-1, 1:-1, 1:-1][~act] = rs.standard_normal(int((~act).sum()))
+    prm = dict(cgpara=0.95, icgtyp=1, cgepsa=1e-15, cgepsr=1e-10, cgdiv=1e30, icgmax=500)
+    y = rs.standard_normal((ni, nj, nk))
+    print(f"packed sweeps {shape}", flush=True)
+    _milu_check(pkg, mat, indc, prm, "SWEEP_PIPELINED", [y, mat["BB"], y])
