@@ -174,7 +174,7 @@ int cad_create(int numi, int numj, int numk, int numb, int device, cad_ctx **out
     rc = rc ? rc : dalloc(&c->xx, 6 * (size_t)numi);
     rc = rc ? rc : dalloc(&c->yy, 6 * (size_t)numj);
     rc = rc ? rc : dalloc(&c->zz, 6 * (size_t)numk);
-    rc = rc ? rc : dalloc(&c->red_partial, 4 * (size_t)REDUCE_BLOCKS);
+    rc = rc ? rc : dalloc(&c->red_partial, REDUCE_SLOTS * (size_t)REDUCE_BLOCKS);
     rc = rc ? rc : dalloc(&c->red_out, 16);
     rc = rc ? rc : dalloc(&c->ksc, 32);
     rc = rc ? rc : dalloc(&c->act_rng, 2);
@@ -194,6 +194,11 @@ int cad_create(int numi, int numj, int numk, int numb, int device, cad_ctx **out
         cad_destroy(c);
         return CAD_ERR_HIP;
     }
+    void *rec = nullptr;
+    if (hipHostGetDevicePointer(&rec, c->host_red, 0) == hipSuccess)
+        c->host_rec = static_cast<double *>(rec) + CAD_REC;
+    else
+        (void)hipGetLastError();
     if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess) {
         cad_set_error("hipStreamCreate failed");
         cad_destroy(c);

@@ -125,6 +125,8 @@ inline dim3 cell_grid(const Dims &d)
 // writes one partial, one block sums the partials in index order.
 constexpr int REDUCE_BLOCKS = 1024;
 constexpr int REDUCE_THREADS = 256;
+constexpr int REDUCE_SLOTS = 6;   // products whose partials are kept apart
+constexpr int CAD_REC = 8;        // first double of the solve's record in host_red
 
 // One level of the multigrid (cad_mg.hip): a grid with one ghost layer, its
 // 7-point rows (inactive rows AD = 1, no couplings), the level's unknowns and
@@ -186,12 +188,13 @@ struct cad_ctx {
     // VOF work: F fluxes
     double *flf[3];
     // scratch for reductions and counters
-    double *red_partial;    // REDUCE_BLOCKS * 4
+    double *red_partial;    // REDUCE_BLOCKS * REDUCE_SLOTS
     double *red_out;        // 16 results
     double *ksc;            // BiCGSTAB scalars on the device (32 slots)
     unsigned long long *act_rng;   // [n0, n1) of the active cells of the current solve
     int *icount;            // 16 int counters
-    double *host_red;       // pinned mirror of red_out
+    double *host_red;       // pinned mirror of red_out; record of the solve's stop test at CAD_REC
+    double *host_rec;       // the record's device address (null: host_red is not pinned)
     int *host_cnt;          // pinned mirror of icount
     // timers
     hipEvent_t ev[16];
@@ -320,12 +323,12 @@ void cad_sweep_free(cad_ctx *c);
 unsigned long long cad_sweep_bytes(const cad_ctx *c);
 int cad_sweep_bind(cad_ctx *c, char *base, unsigned long long bytes, unsigned seq);
 int cad_sweep_dcmp(cad_ctx *c, double u, int *npos_host);
-int cad_sweep_minv(cad_ctx *c, double *x, const double *y);
+int cad_sweep_minv(cad_ctx *c, double *x, const double *y, const double *stop);
 int cad_sweep_status(cad_ctx *c, int *code);
 int cad_wave_alloc(cad_ctx *c);
 void cad_wave_sweep_free(cad_ctx *c);
 int cad_wave_pack(cad_ctx *c);
-int cad_wave_minv(cad_ctx *c, double *x, const double *y);
+int cad_wave_minv(cad_ctx *c, double *x, const double *y, const double *stop);
 int cad_milu_factor_impl(cad_ctx *c, int *npos);
 int cad_poisson_residual_impl(cad_ctx *c, double *rel);
 int cad_poisson_residual_x(cad_ctx *c, const double *x, double *rel);

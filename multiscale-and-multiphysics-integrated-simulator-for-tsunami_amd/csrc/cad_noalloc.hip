@@ -164,7 +164,7 @@ extern "C" int cad_m1bcgs_noalloc(void *stream, const double *ad, const double *
     c.lpk = c.lpj + CAD_NOALLOC_MAX_CELLS;
     char *q = p + LP_BYTES;
     c.red_partial = reinterpret_cast<double *>(q);
-    q += align256(4ull * REDUCE_BLOCKS * sizeof(double));
+    q += align256((unsigned long long)REDUCE_SLOTS * REDUCE_BLOCKS * sizeof(double));
     c.red_out = reinterpret_cast<double *>(q);
     q += align256(16 * sizeof(double));
     c.ksc = reinterpret_cast<double *>(q);
@@ -173,7 +173,7 @@ extern "C" int cad_m1bcgs_noalloc(void *stream, const double *ad, const double *
     q += align256(2 * sizeof(unsigned long long));
     c.icount = reinterpret_cast<int *>(q);
     q += align256((16 + 2 * 1024) * sizeof(int));
-    static_assert(align256(4ull * REDUCE_BLOCKS * 8) + 3 * 256 + align256((16 + 2048) * 4) <=
+    static_assert(align256((unsigned long long)REDUCE_SLOTS * REDUCE_BLOCKS * 8) + 3 * 256 + align256((16 + 2048) * 4) <=
                       SMALL_BYTES, "small scratch arrays");
     c.host_red = s.host_red;
     c.host_cnt = s.host_cnt;

@@ -13,6 +13,8 @@
 #include "cad_common.h"
 
 #include <cmath>
+#include <cstring>
+#include <utility>
 
 namespace {
 
@@ -195,8 +197,11 @@ __global__ void k_bkwd_plane(Dims d, Plane pl, const double *__restrict__ dd,
 // BiCGSTAB scalars live in a small device array (slots SC_*), so the only
 // value the host reads per iteration is (R,R) for the stop test.
 enum { SC_S = 0, SC_W1, SC_ALPHA, SC_W1B, SC_W2, SC_OMEGA, SC_XN, SC_W1C, SC_BETA, SC_BN, SC_N,
-       SC_TRR = 20, SC_TBB = 21 };
-enum { RED_PLAIN = 0, RED_ALPHA, RED_OMEGA, RED_BETA };
+       SC_TRR = 20, SC_TBB = 21, SC_DONE = 22, SC_S1 = 23 };
+// partial sums of the iteration's products, each read by the kernel after
+// next: (r0, ap); (s, ae) and (ae, ae); (r, r) and (r0, r).  Slot 0 is the
+// generic reductions'.
+enum { PS_W1 = 1, PS_OM = 2, PS_XR = 4 };
 constexpr int VEC_BLOCKS = 2048;
 
 // [n0, n1) of the active cells; rng must hold {nc, 0} on entry
@@ -228,8 +233,9 @@ __global__ void __launch_bounds__(256) k_active_range(long long nc, const int *_
     }
 }
 
-__global__ void k_range_init(unsigned long long *rng, long long nc)
+__global__ void k_range_init(unsigned long long *rng, long long nc, double *sc)
 {
+    sc[SC_DONE] = 0.0;
     rng[0] = (unsigned long long)nc;
     rng[1] = 0;
 }
@@ -287,8 +293,9 @@ __global__ void __launch_bounds__(REDUCE_THREADS) k_dot(const unsigned long long
                                                         const int *__restrict__ mask,
                                                         const double *__restrict__ x,
                                                         const double *__restrict__ y,
-                                                        double *partial)
+                                                        const double *stop, double *partial)
 {
+    if (stop && *stop != 0.0) return;
     double acc[3] = {0.0, 0.0, 0.0};
     ACTIVE_LOOP(n, rng, REDUCE_BLOCKS) {
         if (mask[n] != -1) acc[0] += x[n] * y[n];
@@ -301,8 +308,9 @@ __global__ void __launch_bounds__(REDUCE_THREADS) k_dot2(const unsigned long lon
                                                          const int *__restrict__ mask,
                                                          const double *__restrict__ r,
                                                          const double *__restrict__ ae,
-                                                         double *partial)
+                                                         const double *stop, double *partial)
 {
+    if (*stop != 0.0) return;
     double acc[3] = {0.0, 0.0, 0.0};
     ACTIVE_LOOP(n, rng, REDUCE_BLOCKS) {
         if (mask[n] != -1) {
@@ -313,19 +321,61 @@ __global__ void __launch_bounds__(REDUCE_THREADS) k_dot2(const unsigned long lon
     block_reduce_store<2>(acc, partial);
 }
 
+// The sums of N products' partials in block order: the same additions as a
+// stride over the blocks and a halving tree.  Every block of a kernel that
+// needs the scalar forms it (8 KB from the L2), which saves the launch between
+// the product and its use.
+template <int N>
+__device__ __forceinline__ void final_sums(const double *__restrict__ partial, double (&s)[N])
+{
+    __shared__ double sh[N][REDUCE_THREADS];
+#pragma unroll
+    for (int q = 0; q < N; q++) {
+        double a = 0.0;
+#pragma unroll
+        for (int b = 0; b < REDUCE_BLOCKS; b += REDUCE_THREADS) a += partial[q * REDUCE_BLOCKS + b + threadIdx.x];
+        sh[q][threadIdx.x] = a;
+    }
+    __syncthreads();
+    const int t = threadIdx.x & 63, q = threadIdx.x >> 6;
+    if (q < N) {
+        double v = (sh[q][t] + sh[q][t + 128]) + (sh[q][t + 64] + sh[q][t + 192]);
+        for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
+        if (t == 0) sh[q][0] = v;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < N; i++) s[i] = sh[i][0];
+}
+
+// a block whose share of the active range is empty
+__device__ __forceinline__ bool idle_block(const unsigned long long *rng)
+{
+    return rng[0] + (unsigned long long)blockIdx.x * blockDim.x >= rng[1];
+}
+
 // x += alpha p + omega r ; r -= omega ae ; partials of (r, r) and (r0, r),
-// vf_m1bcgs.f:205-227
+// vf_m1bcgs.f:204-227, with omega = (r, ae) / (ae, ae) from k_dot2's partials
 __global__ void __launch_bounds__(REDUCE_THREADS) k_update_xr(const unsigned long long *rng,
                                                               const int *__restrict__ mask,
                                                               double *__restrict__ x,
                                                               double *__restrict__ r,
                                                               const double *__restrict__ p,
                                                               const double *__restrict__ ae,
-                                                              const double *__restrict__ r0,
-                                                              const double *__restrict__ sc,
+                                                              const double *__restrict__ r0, double *sc,
+                                                              const double *__restrict__ om_part,
                                                               double *partial)
 {
-    const double alpha = sc[SC_ALPHA], omega = sc[SC_OMEGA];
+    if (sc[SC_DONE] != 0.0) return;
+    if (blockIdx.x != 0 && idle_block(rng)) {
+        if (threadIdx.x < 2) partial[threadIdx.x * REDUCE_BLOCKS + blockIdx.x] = 0.0;
+        return;
+    }
+    const double alpha = sc[SC_ALPHA];
+    double w[2];
+    final_sums<2>(om_part, w);
+    const double omega = w[0] / w[1];
+    if (blockIdx.x == 0 && threadIdx.x == 0) sc[SC_OMEGA] = omega;
     double acc[3] = {0.0, 0.0, 0.0};
     ACTIVE_LOOP(n, rng, REDUCE_BLOCKS) {
         if (mask[n] != -1) {
@@ -339,37 +389,95 @@ __global__ void __launch_bounds__(REDUCE_THREADS) k_update_xr(const unsigned lon
     block_reduce_store<2>(acc, partial);
 }
 
-// Adds the partials of nprod products in block order into sc[slot..], then
-// forms the BiCGSTAB scalar the next kernel needs (vf_m1bcgs.f:179, 204, 229):
-//   RED_ALPHA: alpha = s / w1          RED_OMEGA: omega = w1 / w2
-//   RED_BETA:  beta = w1 alpha / (s omega), then s = w1
-__global__ void __launch_bounds__(REDUCE_THREADS) k_reduce_final(const double *__restrict__ partial,
-                                                                 int nprod, double *sc, int slot,
-                                                                 int mode)
+// s = r - alpha ap and y = A s (vf_m1bcgs.f:179-196), alpha = s0 / (r0, ap) from
+// k_dot's partials; the neighbours' s is formed on the fly from the same
+// operands, so s goes to a buffer of its own and the vector is not read back
+__global__ void __launch_bounds__(REDUCE_THREADS) k_s_ax(Dims d, const unsigned long long *rng,
+                                                         const double *__restrict__ ad,
+                                                         const double *__restrict__ ali,
+                                                         const double *__restrict__ alj,
+                                                         const double *__restrict__ alk,
+                                                         const double *__restrict__ aui,
+                                                         const double *__restrict__ auj,
+                                                         const double *__restrict__ auk,
+                                                         const int *__restrict__ indc, double *sc, int s_slot,
+                                                         const double *__restrict__ w1_part,
+                                                         const double *__restrict__ r,
+                                                         const double *__restrict__ ap,
+                                                         double *__restrict__ s, double *__restrict__ y)
 {
-    __shared__ double sh[REDUCE_THREADS];
-    for (int q = 0; q < nprod; q++) {
-        double a = 0.0;
-        for (int b = threadIdx.x; b < REDUCE_BLOCKS; b += REDUCE_THREADS) a += partial[q * REDUCE_BLOCKS + b];
-        sh[threadIdx.x] = a;
-        __syncthreads();
-        for (int off = REDUCE_THREADS / 2; off > 0; off >>= 1) {
-            if ((int)threadIdx.x < off) sh[threadIdx.x] += sh[threadIdx.x + off];
-            __syncthreads();
-        }
-        if (threadIdx.x == 0) sc[slot + q] = sh[0];
-        __syncthreads();
+    if (sc[SC_DONE] != 0.0 || (blockIdx.x != 0 && idle_block(rng))) return;
+    double w[1];
+    final_sums<1>(w1_part, w);
+    const double alpha = sc[s_slot] / w[0];
+    if (blockIdx.x == 0 && threadIdx.x == 0) sc[SC_ALPHA] = alpha;
+    const long long ni = d.ni, nij = d.nij;
+    auto v = [&](long long n) { return r[n] - alpha * ap[n]; };
+    ACTIVE_LOOP(n, rng, VEC_BLOCKS) {
+        if (indc[n] == -1) continue;
+        const double c = v(n);
+        s[n] = c;
+        y[n] = ad[n] * c + ali[n] * v(n - 1) + alj[n] * v(n - ni) + alk[n] * v(n - nij)
+             + aui[n] * v(n + 1) + auj[n] * v(n + ni) + auk[n] * v(n + nij);
     }
-    if (threadIdx.x == 0) {
-        if (mode == RED_ALPHA) {
-            sc[SC_ALPHA] = sc[SC_S] / sc[SC_W1];
-        } else if (mode == RED_OMEGA) {
-            sc[SC_OMEGA] = sc[SC_W1B] / sc[SC_W2];
-        } else if (mode == RED_BETA) {
-            sc[SC_BETA] = sc[SC_W1C] * sc[SC_ALPHA] / (sc[SC_S] * sc[SC_OMEGA]);
-            sc[SC_S] = sc[SC_W1C];
+}
+
+// The stop test on (r, r) from k_update_xr's partials (SC_DONE, and the record
+// rec = {(r, r), tag} in host memory), and unless it stops p' = r + beta (p -
+// omega ap) and y = A p' (vf_m1bcgs.f:229-238, 163-170), beta = (r0, r) alpha /
+// (s0 omega).  Stops at (r, r) <= thr and above div2; thr < 0 never stops.
+__global__ void __launch_bounds__(REDUCE_THREADS) k_p_ax(Dims d, const unsigned long long *rng,
+                                                         const double *__restrict__ ad,
+                                                         const double *__restrict__ ali,
+                                                         const double *__restrict__ alj,
+                                                         const double *__restrict__ alk,
+                                                         const double *__restrict__ aui,
+                                                         const double *__restrict__ auj,
+                                                         const double *__restrict__ auk,
+                                                         const int *__restrict__ indc, double *sc, int s_slot,
+                                                         int s_next, double thr, double div2, double *rec, double tag,
+                                                         const double *__restrict__ xr_part,
+                                                         const double *__restrict__ r,
+                                                         const double *__restrict__ p,
+                                                         const double *__restrict__ ap,
+                                                         double *__restrict__ pn, double *__restrict__ y)
+{
+    if (blockIdx.x != 0 && idle_block(rng)) return;
+    double w[2];
+    final_sums<2>(xr_part, w);
+    const bool stop = thr >= 0.0 && (w[0] <= thr || w[0] > div2);
+    const double omega = sc[SC_OMEGA];
+    const double beta = w[1] * sc[SC_ALPHA] / (sc[s_slot] * omega);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        sc[SC_XN] = w[0];
+        sc[SC_DONE] = stop ? 1.0 : 0.0;
+        sc[s_next] = w[1];
+        if (rec) {
+            __hip_atomic_store(rec, w[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            __hip_atomic_store(rec + 1, tag, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
         }
     }
+    if (stop) return;
+    const long long ni = d.ni, nij = d.nij;
+    auto v = [&](long long n) { return r[n] + beta * (p[n] - omega * ap[n]); };
+    ACTIVE_LOOP(n, rng, VEC_BLOCKS) {
+        if (indc[n] == -1) continue;
+        const double c = v(n);
+        pn[n] = c;
+        y[n] = ad[n] * c + ali[n] * v(n - 1) + alj[n] * v(n - ni) + alk[n] * v(n - nij)
+             + aui[n] * v(n + 1) + auj[n] * v(n + ni) + auk[n] * v(n + nij);
+    }
+}
+
+// the generic reductions' sums in block order into sc[slot..]
+template <int N>
+__global__ void __launch_bounds__(REDUCE_THREADS) k_reduce_final(const double *__restrict__ partial, double *sc,
+                                                                 int slot)
+{
+    double s[N];
+    final_sums<N>(partial, s);
+    if (threadIdx.x == 0)
+        for (int q = 0; q < N; q++) sc[slot + q] = s[q];
 }
 
 // ------------------------------------------------------------- vector ops
@@ -405,29 +513,6 @@ __global__ void __launch_bounds__(256) k_init_rp(const unsigned long long *rng, 
             rr[n] = r0[n];
             pp[n] = r0[n];
         }
-    }
-}
-
-// r -= alpha ap (active), vf_m1bcgs.f:181-189
-__global__ void __launch_bounds__(256) k_axpy_neg(const unsigned long long *rng, const int *__restrict__ mask,
-                                                  const double *__restrict__ sc,
-                                                  const double *__restrict__ ap, double *r)
-{
-    const double alpha = sc[SC_ALPHA];
-    ACTIVE_LOOP(n, rng, VEC_BLOCKS) {
-        if (mask[n] != -1) r[n] = r[n] - alpha * ap[n];
-    }
-}
-
-// p = r + beta (p - omega ap) (active), vf_m1bcgs.f:230-238
-__global__ void __launch_bounds__(256) k_update_p(const unsigned long long *rng, const int *__restrict__ mask,
-                                                  const double *__restrict__ sc,
-                                                  const double *__restrict__ r,
-                                                  const double *__restrict__ ap, double *p)
-{
-    const double beta = sc[SC_BETA], omega = sc[SC_OMEGA];
-    ACTIVE_LOOP(n, rng, VEC_BLOCKS) {
-        if (mask[n] != -1) p[n] = r[n] + beta * (p[n] - omega * ap[n]);
     }
 }
 
@@ -507,9 +592,9 @@ static int sweep_dcmp(cad_ctx *c, double u, int *npos_host)
 }
 
 // x = M^-1 y  (vf_mzminv.f:38-41)
-static int minv_launch(cad_ctx *c, double *x, const double *y)
+static int minv_launch(cad_ctx *c, double *x, const double *y, const double *stop)
 {
-    if (c->sweep_schedule != CAD_SWEEP_HYPERPLANE) return cad_sweep_minv(c, x, y);
+    if (c->sweep_schedule != CAD_SWEEP_HYPERPLANE) return cad_sweep_minv(c, x, y, stop);
     const Dims &d = c->d;
     const int hmin = 6, hmax = (d.ni - 1) + (d.nj - 1) + (d.nk - 1);
     for (int h = hmin; h <= hmax; h++) {
@@ -530,10 +615,11 @@ static int minv_launch(cad_ctx *c, double *x, const double *y)
     return CAD_OK;
 }
 
-static int apply_minv(cad_ctx *c, double *x, const double *y)
+// stop: the sweeps do nothing if *stop is not 0 (packed sweeps only)
+static int apply_minv(cad_ctx *c, double *x, const double *y, const double *stop = nullptr)
 {
     int rc = cad_kt_begin(c, CAD_KT_MINV);
-    if (!rc) rc = minv_launch(c, x, y);
+    if (!rc) rc = minv_launch(c, x, y, stop);
     if (!rc) rc = cad_kt_end(c, CAD_KT_MINV, 0.0);
     return rc;
 }
@@ -552,21 +638,23 @@ static int apply_a(cad_ctx *c, const double *x, double *y)
     return CAD_OK;
 }
 
-// partials of nprod products in red_partial -> sc[slot..] (+ scalar mode)
-static int reduce_to(cad_ctx *c, int nprod, int slot, int mode)
+// partials of nprod products in red_partial -> sc[slot..]
+static int reduce_to(cad_ctx *c, int nprod, int slot)
 {
-    hipLaunchKernelGGL(k_reduce_final, dim3(1), dim3(REDUCE_THREADS), 0, c->stream, c->red_partial,
-                       nprod, c->ksc, slot, mode);
+    if (nprod == 1)
+        hipLaunchKernelGGL(k_reduce_final<1>, dim3(1), dim3(REDUCE_THREADS), 0, c->stream, c->red_partial, c->ksc, slot);
+    else
+        hipLaunchKernelGGL(k_reduce_final<2>, dim3(1), dim3(REDUCE_THREADS), 0, c->stream, c->red_partial, c->ksc, slot);
     CAD_CHECK(hipGetLastError());
     return CAD_OK;
 }
 
-static int dot_to(cad_ctx *c, const double *x, const double *y, int slot, int mode)
+static int dot_to(cad_ctx *c, const double *x, const double *y, int slot)
 {
     hipLaunchKernelGGL(k_dot, dim3(REDUCE_BLOCKS), dim3(REDUCE_THREADS), 0, c->stream, c->act_rng,
-                       c->f.indc, x, y, c->red_partial);
+                       c->f.indc, x, y, nullptr, c->red_partial);
     CAD_CHECK(hipGetLastError());
-    return reduce_to(c, 1, slot, mode);
+    return reduce_to(c, 1, slot);
 }
 
 // n scalars sc[slot..] -> host
@@ -578,11 +666,40 @@ static int fetch_sc(cad_ctx *c, int slot, int n, double *out)
     return CAD_OK;
 }
 
+// Waits for the record {value, tag} that a kernel of the stream writes to the
+// context's pinned memory.
+static int wait_record(cad_ctx *c, int tag, double *out)
+{
+    const double *rec = c->host_red + CAD_REC;
+    for (unsigned n = 1;; n++) {
+        long long t;
+        __atomic_load((const long long *)(rec + 1), &t, __ATOMIC_ACQUIRE);
+        double v;
+        std::memcpy(&v, &t, sizeof v);
+        if (v == (double)tag) break;
+        if ((n & 0xFFFFu) == 0) {
+            // an error, or a stream that has run dry without the record
+            const hipError_t e = hipStreamQuery(c->stream);
+            if (e == hipErrorNotReady) continue;
+            CAD_CHECK(e);
+            __atomic_load((const long long *)(rec + 1), &t, __ATOMIC_ACQUIRE);
+            std::memcpy(&v, &t, sizeof v);
+            if (v == (double)tag) break;
+            cad_set_error("the solve's stop record did not arrive");
+            return CAD_ERR_HIP;
+        }
+    }
+    long long t;
+    __atomic_load((const long long *)rec, &t, __ATOMIC_RELAXED);
+    std::memcpy(out, &t, sizeof *out);
+    return CAD_OK;
+}
+
 // Generic reduction used outside the solver (VOF sums, CDIV00): partials in
 // red_partial -> n values on the host.
 int cad_reduce_fetch(cad_ctx *c, int n, double *host_out)
 {
-    RET_IF_(reduce_to(c, n, 0, RED_PLAIN));
+    RET_IF_(reduce_to(c, n, 0));
     return fetch_sc(c, 0, n, host_out);
 }
 
@@ -602,7 +719,7 @@ int cad_solve_m1bcgs(cad_ctx *c, double *x0, double *bnorm_out, double *xnorm_ou
     hipLaunchKernelGGL(k_copy, sg, sb, 0, st, nc, x0, c->xw);
     double *zero_vecs[7] = {c->dd, c->yv, c->r0, c->rr, c->pv, c->ap, c->ae};
     for (double *z : zero_vecs) hipLaunchKernelGGL(k_fill, sg, sb, 0, st, nc, z, 0.0);
-    hipLaunchKernelGGL(k_range_init, dim3(1), dim3(1), 0, st, c->act_rng, nc);
+    hipLaunchKernelGGL(k_range_init, dim3(1), dim3(1), 0, st, c->act_rng, nc, c->ksc);
     hipLaunchKernelGGL(k_active_range, dim3(1024), dim3(256), 0, st, nc, mask, c->act_rng);
     CAD_CHECK(hipGetLastError());
     int iter = -1;
@@ -620,12 +737,12 @@ int cad_solve_m1bcgs(cad_ctx *c, double *x0, double *bnorm_out, double *xnorm_ou
     const double epsr2 = c->prm.cgepsr * c->prm.cgepsr;
     const double div2 = c->prm.cgdiv * c->prm.cgdiv;
     RET_IF_(apply_minv(c, c->yv, c->bb));
-    RET_IF_(dot_to(c, c->yv, c->yv, SC_BN, RED_PLAIN));
+    RET_IF_(dot_to(c, c->yv, c->yv, SC_BN));
     iter = 0;
     RET_IF_(apply_a(c, c->xw, c->yv));
     hipLaunchKernelGGL(k_bminus, vg, sb, 0, st, rng, mask, c->bb, c->yv);
     RET_IF_(apply_minv(c, c->r0, c->yv));
-    RET_IF_(dot_to(c, c->r0, c->r0, SC_S, RED_PLAIN));
+    RET_IF_(dot_to(c, c->r0, c->r0, SC_S));
     double init[2];
     RET_IF_(fetch_sc(c, SC_S, 1, &init[0]));
     RET_IF_(fetch_sc(c, SC_BN, 1, &init[1]));
@@ -637,14 +754,14 @@ int cad_solve_m1bcgs(cad_ctx *c, double *x0, double *bnorm_out, double *xnorm_ou
     const bool true_stop = c->true_stop > 0.0;
     double bb2 = 0.0;
     if (true_stop) {
-        RET_IF_(dot_to(c, c->bb, c->bb, SC_TBB, RED_PLAIN));
+        RET_IF_(dot_to(c, c->bb, c->bb, SC_TBB));
         RET_IF_(fetch_sc(c, SC_TBB, 1, &bb2));
     }
     auto true_ok = [&](bool *ok) -> int {
         RET_IF_(apply_a(c, c->xw, c->yv));
         hipLaunchKernelGGL(k_bminus, vg, sb, 0, st, rng, mask, c->bb, c->yv);
         CAD_CHECK(hipGetLastError());
-        RET_IF_(dot_to(c, c->yv, c->yv, SC_TRR, RED_PLAIN));
+        RET_IF_(dot_to(c, c->yv, c->yv, SC_TRR));
         double rr2 = 0.0;
         RET_IF_(fetch_sc(c, SC_TRR, 1, &rr2));
         *ok = rr2 <= c->true_stop * c->true_stop * bb2;
@@ -653,34 +770,98 @@ int cad_solve_m1bcgs(cad_ctx *c, double *x0, double *bnorm_out, double *xnorm_ou
     bool done = xnorm <= bnorm * epsr2 + epsa2;
     if (done && true_stop) RET_IF_(true_ok(&done));
     if (!done) {
-        hipLaunchKernelGGL(k_init_rp, vg, sb, 0, st, rng, mask, c->r0, c->rr, c->pv);
-        for (;;) {
-            iter = iter + 1;
-            if (iter > c->prm.icgmax) break;
-            RET_IF_(apply_a(c, c->pv, c->yv));
-            RET_IF_(apply_minv(c, c->ap, c->yv));
-            RET_IF_(dot_to(c, c->r0, c->ap, SC_W1, RED_ALPHA));
-            hipLaunchKernelGGL(k_axpy_neg, vg, sb, 0, st, rng, mask, c->ksc, c->ap, c->rr);
-            RET_IF_(apply_a(c, c->rr, c->yv));
-            RET_IF_(apply_minv(c, c->ae, c->yv));
-            hipLaunchKernelGGL(k_dot2, rgd, rbd, 0, st, rng, mask, c->rr, c->ae, c->red_partial);
-            RET_IF_(reduce_to(c, 2, SC_W1B, RED_OMEGA));
-            hipLaunchKernelGGL(k_update_xr, rgd, rbd, 0, st, rng, mask, c->xw, c->rr, c->pv, c->ae,
-                               c->r0, c->ksc, c->red_partial);
-            // (R,R) -> SC_XN, (R0,R) -> SC_W1C; beta and the new s on the device
-            RET_IF_(reduce_to(c, 2, SC_XN, RED_BETA));
-            RET_IF_(fetch_sc(c, SC_XN, 1, &xnorm));
-            if (xnorm <= bnorm * epsr2 + epsa2) {
-                if (!true_stop) break;
-                bool ok = false;
-                RET_IF_(true_ok(&ok));
-                if (ok) break;
+        // An iteration is nine launches: p' with y = A p', M^-1 (two), (r0, ap),
+        // s with y = A s, M^-1, the two products for omega, the updates of x
+        // and r; each scalar is formed by the kernel that needs it.  p', ap, s
+        // and ae go to buffers whose contents are dead by then, in turn.
+        //
+        // The stop test is made on the device by the next iteration's first
+        // kernel.  With packed sweeps and a record in pinned memory the host
+        // launches that whole iteration and then reads the record, so the
+        // device does not wait for the host; if it stopped, the iteration's
+        // other kernels return at once.
+        double *r = c->rr, *p = c->pv, *ap = c->ap, *w = c->ae, *y = c->yv;
+        const bool spec = c->ws_packed && c->sweep_schedule != CAD_SWEEP_HYPERPLANE && c->host_rec &&
+                          !(c->kt && c->kt->on);
+        const double *stop = c->ws_packed ? c->ksc + SC_DONE : nullptr;
+        double *part = c->red_partial;
+        const double thr = bnorm * epsr2 + epsa2;
+        int slot = SC_S;
+        if (spec) c->host_red[CAD_REC + 1] = 0.0;
+        hipLaunchKernelGGL(k_init_rp, vg, sb, 0, st, rng, mask, c->r0, r, p);
+        RET_IF_(apply_a(c, p, y));
+        // the part of an iteration after y = A p
+        auto rest = [&]() -> int {
+            RET_IF_(apply_minv(c, ap, y, stop));
+            hipLaunchKernelGGL(k_dot, rgd, rbd, 0, st, rng, mask, c->r0, ap, c->ksc + SC_DONE,
+                               part + PS_W1 * REDUCE_BLOCKS);
+            hipLaunchKernelGGL(k_s_ax, vg, sb, 0, st, d, rng, c->ad, c->ali, c->alj, c->alk, c->aui, c->auj, c->auk,
+                               mask, c->ksc, slot, part + PS_W1 * REDUCE_BLOCKS, r, ap, w, y);
+            // s in w; r is dead and takes ae
+            RET_IF_(apply_minv(c, r, y, stop));
+            hipLaunchKernelGGL(k_dot2, rgd, rbd, 0, st, rng, mask, w, r, c->ksc + SC_DONE,
+                               part + PS_OM * REDUCE_BLOCKS);
+            hipLaunchKernelGGL(k_update_xr, rgd, rbd, 0, st, rng, mask, c->xw, w, p, r, c->r0, c->ksc,
+                               part + PS_OM * REDUCE_BLOCKS, part + PS_XR * REDUCE_BLOCKS);
+            CAD_CHECK(hipGetLastError());
+            std::swap(r, w);
+            return CAD_OK;
+        };
+        // the stop test, p' and y = A p'; the new p in the old ae's buffer
+        auto next_p = [&](double limit, int tag) -> int {
+            const int nx = slot == SC_S ? SC_S1 : SC_S;
+            hipLaunchKernelGGL(k_p_ax, vg, sb, 0, st, d, rng, c->ad, c->ali, c->alj, c->alk, c->aui, c->auj, c->auk, mask,
+                               c->ksc, slot, nx, limit, div2, spec ? c->host_rec : nullptr, (double)tag,
+                               part + PS_XR * REDUCE_BLOCKS, r, p, ap, w, y);
+            CAD_CHECK(hipGetLastError());
+            return CAD_OK;
+        };
+        iter = 1;
+        if (iter <= c->prm.icgmax) RET_IF_(rest());
+        while (iter <= c->prm.icgmax) {
+            RET_IF_(next_p(thr, iter));
+            // the buffers and the scalar slot as the next iteration has them; the
+            // current ones if it does not take place
+            double *const p0 = p, *const w0 = w;
+            const int slot0 = slot;
+            const bool ahead = spec && iter < c->prm.icgmax;
+            auto advance = [&]() {
+                std::swap(p, w);
+                slot = slot == SC_S ? SC_S1 : SC_S;
+            };
+            double *const r1 = r, *const ap1 = ap;
+            if (ahead) {
+                advance();
+                RET_IF_(rest());
             }
-            if (xnorm > div2) {
+            if (spec)
+                RET_IF_(wait_record(c, iter, &xnorm));
+            else
+                RET_IF_(fetch_sc(c, SC_XN, 1, &xnorm));
+            if (xnorm <= thr) {
+                bool ok = true;
+                if (true_stop) RET_IF_(true_ok(&ok));
+                if (ok) break;
+                // the true residual does not hold yet: this iteration again,
+                // without the test
+                p = p0;
+                w = w0;
+                r = r1;
+                ap = ap1;
+                slot = slot0;
+                if (iter < c->prm.icgmax) {
+                    RET_IF_(next_p(-1.0, iter));
+                    advance();
+                    RET_IF_(rest());
+                }
+            } else if (xnorm > div2) {
                 iter = -2;
                 break;
+            } else if (!ahead) {
+                advance();
+                if (iter < c->prm.icgmax) RET_IF_(rest());
             }
-            hipLaunchKernelGGL(k_update_p, vg, sb, 0, st, rng, mask, c->ksc, c->rr, c->ap, c->pv);
+            iter = iter + 1;
         }
     }
     bnorm = std::sqrt(bnorm);
@@ -709,8 +890,8 @@ int cad_poisson_residual_impl(cad_ctx *c, double *rel)
     RET_IF_(apply_a(c, c->pt, c->yv));
     hipLaunchKernelGGL(k_bminus, vg, sb, 0, c->stream, c->act_rng, c->f.indc, c->bb, c->yv);
     CAD_CHECK(hipGetLastError());
-    RET_IF_(dot_to(c, c->yv, c->yv, SC_S, RED_PLAIN));
-    RET_IF_(dot_to(c, c->bb, c->bb, SC_BN, RED_PLAIN));
+    RET_IF_(dot_to(c, c->yv, c->yv, SC_S));
+    RET_IF_(dot_to(c, c->bb, c->bb, SC_BN));
     double rr = 0.0, bb = 0.0;
     RET_IF_(fetch_sc(c, SC_S, 1, &rr));
     RET_IF_(fetch_sc(c, SC_BN, 1, &bb));
@@ -733,8 +914,8 @@ int cad_poisson_residual_x(cad_ctx *c, const double *x, double *rel)
     RET_IF_(apply_a(c, x, c->yv));
     hipLaunchKernelGGL(k_bminus, vg, sb, 0, c->stream, c->act_rng, c->f.indc, c->bb, c->yv);
     CAD_CHECK(hipGetLastError());
-    RET_IF_(dot_to(c, c->yv, c->yv, SC_S, RED_PLAIN));
-    RET_IF_(dot_to(c, c->bb, c->bb, SC_BN, RED_PLAIN));
+    RET_IF_(dot_to(c, c->yv, c->yv, SC_S));
+    RET_IF_(dot_to(c, c->bb, c->bb, SC_BN));
     double rr = 0.0, bb = 0.0;
     RET_IF_(fetch_sc(c, SC_S, 1, &rr));
     RET_IF_(fetch_sc(c, SC_BN, 1, &bb));
@@ -808,7 +989,7 @@ int cad_time_minv_impl(cad_ctx *c, int reps, float *ms_avg)
 // The active index range [n0, n1) of the context's INDC into act_rng and hr.
 int cad_ext_active_range(cad_ctx *c, unsigned long long hr[2])
 {
-    hipLaunchKernelGGL(k_range_init, dim3(1), dim3(1), 0, c->stream, c->act_rng, c->d.nc);
+    hipLaunchKernelGGL(k_range_init, dim3(1), dim3(1), 0, c->stream, c->act_rng, c->d.nc, c->ksc);
     hipLaunchKernelGGL(k_active_range, dim3(1024), dim3(256), 0, c->stream, c->d.nc, c->f.indc,
                        c->act_rng);
     CAD_CHECK(hipGetLastError());
@@ -833,6 +1014,6 @@ int cad_ext_residual(cad_ctx *c, const double *x, double *y)
 // (x, y) over the active cells, to the host
 int cad_ext_dot(cad_ctx *c, const double *x, const double *y, double *out)
 {
-    RET_IF_(dot_to(c, x, y, SC_S, RED_PLAIN));
+    RET_IF_(dot_to(c, x, y, SC_S));
     return fetch_sc(c, SC_S, 1, out);
 }

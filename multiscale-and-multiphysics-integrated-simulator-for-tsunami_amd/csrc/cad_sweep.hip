@@ -910,9 +910,10 @@ int cad_sweep_dcmp(cad_ctx *c, double u, int *npos_host)
 }
 
 // x = M^-1 y (vf_mzminv.f:38-41): forward then backward sweep, in place on x.
-int cad_sweep_minv(cad_ctx *c, double *x, const double *y)
+// The packed sweeps do nothing if stop is given and *stop is not 0.
+int cad_sweep_minv(cad_ctx *c, double *x, const double *y, const double *stop)
 {
-    if (c->ws_packed) return cad_wave_minv(c, x, y);
+    if (c->ws_packed) return cad_wave_minv(c, x, y, stop);
     FwdOp f;
     f.src[0] = y;
     f.src[1] = c->lpi;

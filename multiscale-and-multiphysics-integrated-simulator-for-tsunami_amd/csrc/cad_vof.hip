@@ -449,17 +449,24 @@ __global__ void __launch_bounds__(REDUCE_THREADS) k_fcut(Dims d, Static s, const
     }
 }
 
-// FSUM and FCUT from k_fcut's partials, compensated, in block order
-__global__ void k_fcut_final(const double *__restrict__ partial, double *out)
+// FSUM and FCUT from k_fcut's partials, compensated, in a fixed order: a wave
+// for each, its lanes over a stride of the blocks, then a halving tree (one
+// thread over all blocks took 46 us)
+__global__ void __launch_bounds__(128) k_fcut_final(const double *__restrict__ partial, double *out)
 {
-    if (threadIdx.x >= 2) return;
-    const int q = threadIdx.x;
+    const int q = threadIdx.x >> 6, t = threadIdx.x & 63;
     double a = 0.0, c = 0.0;
-    for (int b = 0; b < REDUCE_BLOCKS; b++) {
+#pragma unroll 4
+    for (int b = t; b < REDUCE_BLOCKS; b += 64) {
         comp_add(a, c, partial[q * REDUCE_BLOCKS + b]);
         c += partial[(q + 2) * REDUCE_BLOCKS + b];
     }
-    out[q] = a + c;
+    for (int off = 32; off > 0; off >>= 1) {
+        const double b = __shfl_down(a, off, 64), e = __shfl_down(c, off, 64);
+        comp_add(a, c, b);
+        c += e;
+    }
+    if (t == 0) out[q] = a + c;
 }
 
 // Boundary F, vf_bwff.f:33-87 (types FIX and FREE; wave-maker and radiation
@@ -992,7 +999,7 @@ int cad_vof_phase(cad_ctx *c, double *fsum, double *fcut)
     // VF_FCUT01 (vf_f1cal.f:188)
     hipLaunchKernelGGL(k_fcut, dim3(REDUCE_BLOCKS), dim3(REDUCE_THREADS), 0, st, d, s, f.nf, f.ff,
                        c->prm.flower, c->prm.fupper, c->red_partial);
-    hipLaunchKernelGGL(k_fcut_final, dim3(1), dim3(64), 0, st, c->red_partial, c->red_out);
+    hipLaunchKernelGGL(k_fcut_final, dim3(1), dim3(128), 0, st, c->red_partial, c->red_out);
     CAD_CHECK(hipGetLastError());
     CAD_CHECK(hipMemcpyAsync(c->host_red, c->red_out, 2 * sizeof(double), hipMemcpyDeviceToHost, st));
     CAD_CHECK(hipStreamSynchronize(st));
@@ -1054,7 +1061,7 @@ int cad_init_phase(cad_ctx *c, double wvlvl, const double *uvw, int flags, doubl
     RET_IF(cad_launch_bwffsf(c));
     hipLaunchKernelGGL(k_fcut, dim3(REDUCE_BLOCKS), dim3(REDUCE_THREADS), 0, st, d, s, f.nf, f.ff,
                        c->prm.flower, c->prm.fupper, c->red_partial);
-    hipLaunchKernelGGL(k_fcut_final, dim3(1), dim3(64), 0, st, c->red_partial, c->red_out);
+    hipLaunchKernelGGL(k_fcut_final, dim3(1), dim3(128), 0, st, c->red_partial, c->red_out);
     CAD_CHECK(hipGetLastError());
     CAD_CHECK(hipMemcpyAsync(c->host_red, c->red_out, 2 * sizeof(double), hipMemcpyDeviceToHost, st));
     CAD_CHECK(hipStreamSynchronize(st));

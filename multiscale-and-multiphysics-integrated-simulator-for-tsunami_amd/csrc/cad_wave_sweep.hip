@@ -89,6 +89,7 @@ struct WCtl {
     unsigned long long base;
     unsigned seq;
     int *err;
+    const double *stop;             // not null and not 0: nothing to do
 };
 
 // forward: LPI, LPJ, LPK packed (LPI = MARK on cells that are not active), Y in
@@ -479,7 +480,7 @@ __global__ void __launch_bounds__(64 * waves(NW), 1) k_wave(WGeom g, WCtl c, Op 
     }
     __syncthreads();
     const int tile = __builtin_amdgcn_readfirstlane(sm.tile);
-    if (tile < 0) return;
+    if (tile < 0 || (c.stop && *c.stop != 0.0)) return;
     const int2 rg = c.range[tile];
     if (rg.x > rg.y) return;
     const int bj = tile % g.ntj, bk = tile / g.ntj;
@@ -745,7 +746,7 @@ struct cad_wsweep {
 
 namespace {
 
-WCtl wctl(const cad_ctx *c)
+WCtl wctl(const cad_ctx *c, const double *stop)
 {
     const cad_wsweep *ws = c->ws;
     WCtl s;
@@ -758,17 +759,18 @@ WCtl wctl(const cad_ctx *c)
     s.base = c->sw_base;
     s.seq = c->sw_seq;
     s.err = c->sw_err;
+    s.stop = stop;
     return s;
 }
 
 template <class Op>
-int wave_launch(cad_ctx *c, const Op &op)
+int wave_launch(cad_ctx *c, const Op &op, const double *stop)
 {
     const cad_wsweep *ws = c->ws;
     if (ws->nw == 1)
-        hipLaunchKernelGGL((k_wave<Op, 1>), dim3(ws->g.ntiles), dim3(64 * waves(1)), 0, c->stream, ws->g, wctl(c), op);
+        hipLaunchKernelGGL((k_wave<Op, 1>), dim3(ws->g.ntiles), dim3(64 * waves(1)), 0, c->stream, ws->g, wctl(c, stop), op);
     else
-        hipLaunchKernelGGL((k_wave<Op, 2>), dim3(ws->g.ntiles), dim3(64 * waves(2)), 0, c->stream, ws->g, wctl(c), op);
+        hipLaunchKernelGGL((k_wave<Op, 2>), dim3(ws->g.ntiles), dim3(64 * waves(2)), 0, c->stream, ws->g, wctl(c, stop), op);
     CAD_CHECK(hipGetLastError());
     c->sw_base += (unsigned long long)ws->g.ntiles;
     c->sw_seq += 1;
@@ -890,8 +892,9 @@ int cad_wave_pack(cad_ctx *c)
     return CAD_OK;
 }
 
-// x = M^-1 y (vf_mzminv.f:38-41); x may be y.
-int cad_wave_minv(cad_ctx *c, double *x, const double *y)
+// x = M^-1 y (vf_mzminv.f:38-41); x may be y.  Does nothing if stop is given and
+// *stop is not 0.
+int cad_wave_minv(cad_ctx *c, double *x, const double *y, const double *stop)
 {
     const cad_wsweep *ws = c->ws;
     WFwd f;
@@ -899,12 +902,12 @@ int cad_wave_minv(cad_ctx *c, double *x, const double *y)
     f.nat_in = y;
     f.pk_out = ws->pk[7];
     f.nat_out = x;
-    if (int rc = wave_launch(c, f)) return rc;
+    if (int rc = wave_launch(c, f, stop)) return rc;
     WBwd b;
     for (int q = 0; q < 4; q++) b.src[q] = ws->pk[3 + q];
     b.src[4] = ws->pk[7];
     b.nat_in = y;
     b.pk_out = ws->pk[7];
     b.nat_out = x;
-    return wave_launch(c, b);
+    return wave_launch(c, b, stop);
 }
