@@ -684,9 +684,10 @@ __global__ void __launch_bounds__(64 * NW) k_wave_range(WGeom g, const int2 *__r
     if (l == 0) range[tile] = shi[0] < 0 ? make_int2(1, 0) : make_int2(slo[0], shi[0]);
 }
 
-// The operands of both sweeps in walking order, 64 diagonals of one wave per
-// block: lines are read along I, turned in LDS and written a diagonal pair at a
-// time.  LPI = ALI*DD(n-1), LPJ = ALJ*DD(n-NI), LPK = ALK*DD(n-NIJ), the products
+// The operands of both sweeps in walking order, 64 diagonals of one wave and one
+// operand per block: lines are read along I, turned in LDS and written a
+// diagonal pair at a time (the seven operands one after the other took 62 us on
+// 64x16x48, side by side 12).  LPI = ALI*DD(n-1), LPJ = ALJ*DD(n-NI), LPK = ALK*DD(n-NIJ), the products
 // the reference forms before multiplying by X.
 struct PackArgs {
     const double *ali, *alj, *alk, *aui, *auj, *auk, *dd;
@@ -706,8 +707,8 @@ __global__ void __launch_bounds__(256) k_wave_pack(WGeom g, const int2 *__restri
     const double *src[7] = {a.ali, a.alj, a.alk, a.aui, a.auj, a.auk, a.dd};
     const long long back[3] = {1, g.ni, g.nij};
     const long long np = g.nd / 2;
-#pragma unroll 1
-    for (int q = 0; q < 7; q++) {
+    {
+        const int q = blockIdx.z;
         for (int L = wv; L < 64; L += 4) {
             const int jl = L & 15, kl = L >> 4;
             const int j = 1 + bj * TJ + jl, k = 1 + (bk * NW + w) * TKW + kl, i = d0 + ii - jl - DK * kl;
@@ -719,7 +720,6 @@ __global__ void __launch_bounds__(256) k_wave_pack(WGeom g, const int2 *__restri
             }
             t[L][ii] = v;
         }
-        __syncthreads();
         for (int p = wv; p < 32; p += 4)
             if (d0 / 2 + p < np)
                 a.out[q][((long long)wt * np + d0 / 2 + p) * 64 + ii] = v2d{t[ii][2 * p], t[ii][2 * p + 1]};
@@ -883,7 +883,7 @@ int cad_wave_pack(cad_ctx *c)
     a.auk = c->auk;
     a.dd = c->dd;
     for (int q = 0; q < 7; q++) a.out[q] = ws->pk[q];
-    const dim3 pg(g.ntiles * ws->nw, (g.nd + 63) / 64);
+    const dim3 pg(g.ntiles * ws->nw, (g.nd + 63) / 64, 7);
     if (ws->nw == 1)
         hipLaunchKernelGGL(k_wave_pack<1>, pg, dim3(256), 0, c->stream, g, ws->range, c->f.indc, a);
     else
