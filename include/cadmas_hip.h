@@ -411,7 +411,7 @@ void vf_vpsol_(double *dbuf, const double *ad, const double *ali, const double *
  * that overlap on one GPU share that array and race.  Returns CAD_OK, or a
  * negative code with the cause in cad_last_error(). */
 #define CAD_NOALLOC_MAX_CELLS 2097152ull                                   /* 2^21 */
-#define CAD_NOALLOC_SCRATCH_BYTES ((72ull << 20) + (64ull << 10))          /* 72.06 MiB */
+#define CAD_NOALLOC_SCRATCH_BYTES ((296ull << 20) + (64ull << 10))         /* 296.06 MiB */
 int cad_m1bcgs_noalloc(void *stream, const double *ad, const double *ali, const double *alj,
                        const double *alk, const double *aui, const double *auj,
                        const double *auk, const double *bb, double *x0, double *dd, double *xw,

@@ -326,6 +326,8 @@ int cad_sweep_dcmp(cad_ctx *c, double u, int *npos_host);
 int cad_sweep_minv(cad_ctx *c, double *x, const double *y, const double *stop);
 int cad_sweep_status(cad_ctx *c, int *code);
 int cad_wave_alloc(cad_ctx *c);
+int cad_wave_bind(cad_ctx *c, struct cad_wsweep **store, char *pk, size_t pk_bytes, char *ctl, size_t ctl_bytes,
+                  char *mb, size_t mb_bytes);
 void cad_wave_sweep_free(cad_ctx *c);
 int cad_wave_pack(cad_ctx *c);
 int cad_wave_minv(cad_ctx *c, double *x, const double *y, const double *stop);

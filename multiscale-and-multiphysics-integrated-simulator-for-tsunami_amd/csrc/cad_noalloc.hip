@@ -10,7 +10,8 @@
 // solver's vectors exactly as they do in the reference.  Everything else the
 // solve needs -- the MILU products LPI/LPJ/LPK, the reduction partials and
 // scalars, the active index range, the counters, the sweeps' tile orders,
-// ranges, mailboxes, ticket and error flag -- lives in one file-scope device
+// ranges, mailboxes, ticket and error flag, the packed sweeps' operands where
+// they fit -- lives in one file-scope device
 // array, `scratch`, of CAD_NOALLOC_SCRATCH_BYTES.  Each GPU the library runs
 // on holds its own copy until the process ends.  Its device address is taken
 // once per device with hipGetSymbolAddress and used for every access from the
@@ -32,7 +33,12 @@ namespace {
 constexpr int MAX_DEVICES = 64;
 constexpr unsigned long long LP_BYTES = 3ull * CAD_NOALLOC_MAX_CELLS * 8ull;
 constexpr unsigned long long SMALL_BYTES = 64ull << 10;
-constexpr unsigned long long SWEEP_BYTES = CAD_NOALLOC_SCRATCH_BYTES - LP_BYTES - SMALL_BYTES;
+constexpr unsigned long long SWEEP_BYTES = 24ull << 20;
+// the packed sweeps' arrays behind them: mailboxes, orders and ranges, operands
+constexpr unsigned long long WMB_AT = LP_BYTES + SMALL_BYTES + SWEEP_BYTES, WMB_BYTES = 24ull << 20;
+constexpr unsigned long long WCTL_AT = WMB_AT + WMB_BYTES, WCTL_BYTES = 8ull << 20;
+constexpr unsigned long long WPK_AT = WCTL_AT + WCTL_BYTES, WPK_BYTES = CAD_NOALLOC_SCRATCH_BYTES - WPK_AT;
+static_assert(CAD_NOALLOC_SCRATCH_BYTES > WPK_AT, "room for the packed operands");
 
 __device__ __align__(256) unsigned char scratch[CAD_NOALLOC_SCRATCH_BYTES];
 
@@ -40,6 +46,7 @@ struct DeviceState {
     bool ready;
     char *ptr;              // device address of this device's scratch
     unsigned seq;           // next sweep sequence number on this device
+    struct cad_wsweep *ws;  // the packed sweeps' places in it
     cad_ctx ctx;            // the solve's view of the caller's arrays and the scratch
     double host_red[16];
     int host_cnt[16];
@@ -67,7 +74,7 @@ int prepare(int dev, hipStream_t st)
     // mailboxes start at sequence number 0 (never a launch's number)
     hipLaunchKernelGGL(k_clear_bytes, dim3(1024), dim3(256), 0, st,
                        reinterpret_cast<unsigned long long *>(ptr + LP_BYTES + SMALL_BYTES),
-                       SWEEP_BYTES / 8);
+                       (SWEEP_BYTES + WMB_BYTES) / 8);
     CAD_CHECK(hipGetLastError());
     CAD_CHECK(hipStreamSynchronize(st));
     s.ptr = ptr;
@@ -126,7 +133,7 @@ extern "C" int cad_m1bcgs_noalloc(void *stream, const double *ad, const double *
     c.d.nij = (long long)ni * nj;
     c.d.nc = nc;
     c.sweep_schedule = CAD_SWEEP_PIPELINED;
-    c.ws_off = true;   // no allocation: the natural-layout sweeps
+    c.ws_off = true;   // no allocation: packed sweeps where they fit the scratch, else the natural-layout ones
     if (cad_sweep_bytes(&c) > SWEEP_BYTES) {
         cad_set_error("cad_m1bcgs_noalloc: the sweeps of %d x %d x %d need %llu bytes of mailboxes, "
                       "more than the %llu reserved", ni, nj, nk, cad_sweep_bytes(&c), SWEEP_BYTES);
@@ -178,6 +185,7 @@ extern "C" int cad_m1bcgs_noalloc(void *stream, const double *ad, const double *
     c.host_red = s.host_red;
     c.host_cnt = s.host_cnt;
     int rc = cad_sweep_bind(&c, p + LP_BYTES + SMALL_BYTES, SWEEP_BYTES, s.seq);
+    if (rc == CAD_OK) rc = cad_wave_bind(&c, &s.ws, p + WPK_AT, WPK_BYTES, p + WCTL_AT, WCTL_BYTES, p + WMB_AT, WMB_BYTES);
     if (rc == CAD_OK) rc = cad_solve_m1bcgs(&c, x0, bnorm, xnorm, iter);
     // the sequence numbers this call used stay behind in the mailboxes
     s.seq = c.sw_seq;

@@ -48,4 +48,16 @@ __device__ __forceinline__ void mb_store(__amdgpu_buffer_rsrc_t r, unsigned off,
     __builtin_amdgcn_raw_buffer_store_b128(e, r, off, 0, CPOL_DEVICE);
 }
 
+// The tiles in the dependency order of the sweeps: by anti-diagonal bj + bk,
+// then by bj.
+__global__ void k_tile_order(int ntj, int ntk, int *order)
+{
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= ntj * ntk) return;
+    const int bj = t % ntj, diag = t % ntj + t / ntj;
+    int pos = 0;
+    for (int s = 0; s < diag; s++) pos += min(ntj - 1, s) - max(0, s - (ntk - 1)) + 1;
+    order[pos + bj - max(0, diag - (ntk - 1))] = t;
+}
+
 }  // namespace

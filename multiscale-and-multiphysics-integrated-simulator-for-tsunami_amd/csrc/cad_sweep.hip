@@ -736,18 +736,6 @@ int cad_sweep_alloc(cad_ctx *c)
 
 namespace {
 
-// Position of each tile in the dependency order that cad_sweep_alloc sorts on
-// the host: by anti-diagonal bj + bk, then by bj.
-__global__ void k_tile_order(int ntj, int ntk, int *order)
-{
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= ntj * ntk) return;
-    const int bj = t % ntj, diag = t % ntj + t / ntj;
-    int pos = 0;
-    for (int s = 0; s < diag; s++) pos += min(ntj - 1, s) - max(0, s - (ntk - 1)) + 1;
-    order[pos + bj - max(0, diag - (ntk - 1))] = t;
-}
-
 __global__ void k_clear_u64(unsigned long long *p, int n)
 {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;

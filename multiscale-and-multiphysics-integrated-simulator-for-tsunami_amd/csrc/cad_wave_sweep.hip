@@ -54,10 +54,8 @@
 #include "cad_common.h"
 #include "cad_sweep.h"
 
-#include <algorithm>
 #include <climits>
-#include <cstring>
-#include <vector>
+#include <new>
 
 namespace {
 
@@ -720,10 +718,10 @@ __global__ void __launch_bounds__(256) k_wave_pack(WGeom g, const int2 *__restri
             }
             t[L][ii] = v;
         }
+        __syncthreads();
         for (int p = wv; p < 32; p += 4)
             if (d0 / 2 + p < np)
                 a.out[q][((long long)wt * np + d0 / 2 + p) * 64 + ii] = v2d{t[ii][2 * p], t[ii][2 * p + 1]};
-        __syncthreads();
     }
 }
 
@@ -742,6 +740,7 @@ struct cad_wsweep {
     int2 *range, *lines;
     v4u *mb;
     unsigned mb_bytes, j_base;
+    size_t pk_bytes;        // of one packed operand
 };
 
 namespace {
@@ -779,16 +778,16 @@ int wave_launch(cad_ctx *c, const Op &op, const double *stop)
 
 }  // namespace
 
-// Allocates the packed sweeps' arrays; leaves c->ws null (the caller then uses
-// the natural-layout sweeps) when their offsets exceed 31 bits or the
-// memory is not there.
-int cad_wave_alloc(cad_ctx *c)
+namespace {
+
+struct WSizes {
+    size_t pk, ctl, mb;   // bytes of the packed operands, of order, ranges and lines, of the mailboxes
+};
+
+// the geometry and the arrays' sizes for a grid; false where 32-bit offsets do
+// not reach
+bool wave_geometry(const Dims &d, cad_wsweep *ws, WSizes *z)
 {
-    if (c->ws || c->ws_off) return CAD_OK;
-    c->ws_off = true;
-    const Dims &d = c->d;
-    cad_wsweep *ws = new (std::nothrow) cad_wsweep();
-    if (!ws) return CAD_OK;
     // One walking wave a workgroup has its CU's cache bandwidth to itself, two
     // share it but hand over in LDS what one would through memory.  Walks of
     // few steps are bound by the handovers, long or wide ones by the steps: on
@@ -807,52 +806,85 @@ int cad_wave_alloc(cad_ctx *c)
     g.nd = (d.ni + SKMAX + S - 1) / S * S;
     const unsigned long long nt = (unsigned long long)g.ntj * g.ntk;
     const unsigned long long kb = nt * (g.nd + 2 * KPAD) * TJ * 16, jb = nt * nw * (g.nd + 2 * JPAD) * TKW * 16;
-    if (kb + jb > 0x7FFFFFF0ull || (unsigned long long)d.nc * 8 > 0xFFFFFFF0ull) {
-        delete ws;
-        return CAD_OK;
-    }
+    if (kb + jb > 0x7FFFFFF0ull || (unsigned long long)d.nc * 8 > 0xFFFFFFF0ull) return false;
     g.ntiles = (int)nt;
     ws->mb_bytes = (unsigned)(kb + jb);
     ws->j_base = (unsigned)kb;
-    const size_t pkb = align256(nt * nw * (size_t)g.nd * 64 * 8), ob = align256(nt * sizeof(int));
-    const size_t rb = align256(nt * sizeof(int2)), lb = align256((size_t)(d.nj - 2) * (d.nk - 2) * sizeof(int2));
-    const size_t total = 8 * pkb + ob + rb + lb + align256(ws->mb_bytes);
-    if (hipMalloc((void **)&ws->mem, total) != hipSuccess) {
+    ws->pk_bytes = align256(nt * nw * (size_t)g.nd * 64 * 8);
+    z->pk = 8 * ws->pk_bytes;
+    z->ctl = align256(nt * sizeof(int)) + align256(nt * sizeof(int2)) +
+             align256((size_t)(d.nj - 2) * (d.nk - 2) * sizeof(int2));
+    z->mb = align256(ws->mb_bytes);
+    return true;
+}
+
+// the arrays at their places and the tile order
+int wave_place(cad_ctx *c, cad_wsweep *ws, char *pk, char *ctl, char *mb)
+{
+    for (v2d *&q : ws->pk) {
+        q = reinterpret_cast<v2d *>(pk);
+        pk += ws->pk_bytes;
+    }
+    const WGeom &g = ws->g;
+    ws->order = reinterpret_cast<int *>(ctl);
+    ctl += align256(g.ntiles * sizeof(int));
+    ws->range = reinterpret_cast<int2 *>(ctl);
+    ctl += align256(g.ntiles * sizeof(int2));
+    ws->lines = reinterpret_cast<int2 *>(ctl);
+    ws->mb = reinterpret_cast<v4u *>(mb);
+    hipLaunchKernelGGL(k_tile_order, dim3((g.ntiles + 255) / 256), dim3(256), 0, c->stream, g.ntj, g.ntk, ws->order);
+    CAD_CHECK(hipGetLastError());
+    return CAD_OK;
+}
+
+__global__ void k_wave_clear(v4u *p, unsigned n)
+{
+    for (unsigned i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) p[i] = v4u{0, 0, 0, 0};
+}
+
+}  // namespace
+
+// Allocates the packed sweeps' arrays; leaves c->ws null (the caller then uses
+// the natural-layout sweeps) when their offsets exceed 31 bits or the
+// memory is not there.
+int cad_wave_alloc(cad_ctx *c)
+{
+    if (c->ws || c->ws_off) return CAD_OK;
+    c->ws_off = true;
+    cad_wsweep *ws = new (std::nothrow) cad_wsweep();
+    if (!ws) return CAD_OK;
+    WSizes z;
+    if (!wave_geometry(c->d, ws, &z)) {
+        delete ws;
+        return CAD_OK;
+    }
+    if (hipMalloc((void **)&ws->mem, z.pk + z.ctl + z.mb) != hipSuccess) {
         (void)hipGetLastError();
         delete ws;
         return CAD_OK;
     }
-    char *p = ws->mem;
-    for (v2d *&q : ws->pk) {
-        q = reinterpret_cast<v2d *>(p);
-        p += pkb;
-    }
-    ws->order = reinterpret_cast<int *>(p);
-    p += ob;
-    ws->range = reinterpret_cast<int2 *>(p);
-    p += rb;
-    ws->lines = reinterpret_cast<int2 *>(p);
-    p += lb;
-    ws->mb = reinterpret_cast<v4u *>(p);
-    std::vector<int> order((size_t)nt);
-    for (int t = 0; t < g.ntiles; t++) order[t] = t;
-    const int ntj = g.ntj;
-    std::stable_sort(order.begin(), order.end(), [ntj](int a, int b) {
-        const int da = a % ntj + a / ntj, db = b % ntj + b / ntj;
-        if (da != db) return da < db;
-        return a % ntj < b % ntj;
-    });
-    // the entries start below every launch's sequence number
-    if (hipMemcpy(ws->order, order.data(), nt * sizeof(int), hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemset(ws->mb, 0, ws->mb_bytes) != hipSuccess || hipDeviceSynchronize() != hipSuccess) {
-        cad_set_error("packed sweeps: set-up failed");
-        (void)hipFree(ws->mem);
-        delete ws;
-        return CAD_ERR_HIP;
-    }
     c->ws = ws;
     c->ws_off = false;
-    return CAD_OK;
+    // the entries start below every launch's sequence number
+    char *mb = ws->mem + z.pk + z.ctl;
+    hipLaunchKernelGGL(k_wave_clear, dim3(1024), dim3(256), 0, c->stream, reinterpret_cast<v4u *>(mb),
+                       (unsigned)(ws->mb_bytes / 16));
+    return wave_place(c, ws, ws->mem, ws->mem + z.pk, mb);
+}
+
+// The same arrays in memory that the caller owns; leaves c->ws null where they
+// do not fit.  *store is the caller's, made on the first call and kept.  The
+// mailboxes' memory holds nothing but mailbox entries of earlier calls, whose
+// sequence numbers c->sw_seq exceeds (0 at first).
+int cad_wave_bind(cad_ctx *c, cad_wsweep **store, char *pk, size_t pk_bytes, char *ctl, size_t ctl_bytes, char *mb,
+                  size_t mb_bytes)
+{
+    if (!*store) *store = new (std::nothrow) cad_wsweep();
+    WSizes z;
+    if (!*store || !wave_geometry(c->d, *store, &z) || z.pk > pk_bytes || z.ctl > ctl_bytes || z.mb > mb_bytes)
+        return CAD_OK;
+    c->ws = *store;
+    return wave_place(c, *store, pk, ctl, mb);
 }
 
 void cad_wave_sweep_free(cad_ctx *c)
