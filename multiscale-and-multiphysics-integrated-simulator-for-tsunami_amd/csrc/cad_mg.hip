@@ -38,12 +38,11 @@
 // half-sweep that follows it; the coarsest level is smoothed MG_COARSE
 // times.  Every level starts from x = 0, so the first (even) half of its
 // first sweep is x = b/AD, which the kernel that sets b writes at once.  The
-// levels of at most MG_TAIL_CELLS cells run as one workgroup (k_mg_tail), so
-// the small grids cost one launch instead of five per level.
+// coarsest levels run as one workgroup (k_mg_tail), so the small grids cost
+// one launch instead of four per level.
 #include "cad_common.h"
 
 #include <algorithm>
-#include <climits>
 
 #define RET_IF(x)              \
     do {                       \
@@ -56,14 +55,13 @@ namespace {
 
 constexpr float MG_SCALE = 1.8f;
 constexpr int MG_COARSE = 12;
-constexpr long long MG_TAIL_CELLS = 4096;
 
-// position of cell (i,j,k) (1-based, ghosts included) in a level's arrays
+// position of cell (i,j,k) (1-based, ghosts included) in a level's arrays (32
+// bits: a grid of 2^31 cells has more than 500 GB of FP64 arrays)
 template <typename L>
-__device__ __forceinline__ long long pos(const L &v, int i, int j, int k)
+__device__ __forceinline__ int pos(const L &v, int i, int j, int k)
 {
-    const long long line = (long long)v.ld * ((j - 1) + (long long)v.d.nj * (k - 1));
-    return line + (long long)((i + j + k) & 1) * (v.ld >> 1) + ((i - 1) >> 1);
+    return v.ld * ((j - 1) + v.d.nj * (k - 1)) + ((i + j + k) & 1) * (v.ld >> 1) + ((i - 1) >> 1);
 }
 
 __device__ __forceinline__ long long nat(const Dims &d, int i, int j, int k)
@@ -163,19 +161,47 @@ __global__ void __launch_bounds__(256) k_mg_coarsen(MgLevelT<V> F, MgLevelT<V> C
     C.auk[m] = a ? s_uk : (V)0;
 }
 
-// the off-diagonal part of row (i,j,k) at position n
+// A cell's neighbours are all of the other colour: cell i of half-line position
+// q is i = 2q+1+p, and its I neighbours are at positions q-1+p and q+p of its
+// line's other half, its J and K neighbours at q of the other half of their
+// lines.
 template <typename V>
-__device__ __forceinline__ V row_off(const MgLevelT<V> &L, long long n, int i, int j, int k)
+struct Cell {
+    int n, o;      // position of the cell, and of position q of its line's other half
+    int p;
+};
+
+template <typename V>
+__device__ __forceinline__ Cell<V> cell_at(const MgLevelT<V> &L, int q, int i, int j, int k, int color)
 {
-    const V *x = L.x;
-    return L.ali[n] * x[pos(L, i - 1, j, k)] + L.aui[n] * x[pos(L, i + 1, j, k)]
-         + L.alj[n] * x[pos(L, i, j - 1, k)] + L.auj[n] * x[pos(L, i, j + 1, k)]
-         + L.alk[n] * x[pos(L, i, j, k - 1)] + L.auk[n] * x[pos(L, i, j, k + 1)];
+    const int half = L.ld >> 1, line = L.ld * ((j - 1) + L.d.nj * (k - 1));
+    return {line + color * half + q, line + (1 - color) * half + q, i - 2 * q - 1};
 }
 
-// one colour of a Gauss-Seidel sweep: thread x covers position q of its
-// (J,K) line's half of that colour (cell I = 2q+1 or 2q+2), K in [k0, k1]
+// the off-diagonal part of the cell's row
 template <typename V>
+__device__ __forceinline__ V row_off(const MgLevelT<V> &L, const Cell<V> &c)
+{
+    const V *x = L.x;
+    const int lj = L.ld, lk = L.ld * L.d.nj;
+    return L.ali[c.n] * x[c.o - 1 + c.p] + L.aui[c.n] * x[c.o + c.p]
+         + L.alj[c.n] * x[c.o - lj] + L.auj[c.n] * x[c.o + lj]
+         + L.alk[c.n] * x[c.o - lk] + L.auk[c.n] * x[c.o + lk];
+}
+
+// The passes of a V-cycle are bound by HBM bandwidth on grids of millions of
+// cells and by their loads' latency on small ones, where a pass is one round of
+// loads if none waits for another's value.  So the activity is tested when the
+// result is stored (an inactive row's operands are finite and in bounds), and
+// only on levels of more than MG_SKIP_CELLS, whose waves without an active cell
+// are worth skipping, before the loads (SKIP).  Tested first everywhere, the
+// restriction took 6.6 us on 97x61x29 and 35.7 on 512x256x45 cells, the
+// correction 5.7 and 41.5; now 4.6 and 31.7, 3.9 and 29.8.
+constexpr long long MG_SKIP_CELLS = 1 << 20;
+
+// one colour of a Gauss-Seidel sweep: thread x covers position q of its
+// (J,K) line's half of that colour (cell I = 2q+1 or 2q+2), K from k0
+template <typename V, bool SKIP>
 __global__ void __launch_bounds__(256) k_mg_smooth(MgLevelT<V> L, int color, int k0)
 {
     const int j = blockIdx.y * blockDim.y + threadIdx.y + 2;
@@ -184,43 +210,54 @@ __global__ void __launch_bounds__(256) k_mg_smooth(MgLevelT<V> L, int color, int
     const int q = (int)(blockIdx.x * blockDim.x + threadIdx.x);
     const int i = 2 * q + 1 + ((color + 1 + j + k) & 1);
     if (i < 2 || i > L.d.ni - 1) return;
-    const long long n = pos(L, i, j, k);
-    if (!L.act[n]) return;
-    L.x[n] = (L.b[n] - row_off(L, n, i, j, k)) / L.ad[n];
+    const Cell<V> c = cell_at(L, q, i, j, k, color);
+    const bool act = L.act[c.n] != 0;
+    if (SKIP && !act) return;
+    const V x = (L.b[c.n] - row_off(L, c)) / L.ad[c.n];
+    if (act) L.x[c.n] = x;
 }
 
 // Coarse right-hand side = sum of the fine residuals of the block; coarse
 // x = 0.  It follows the odd half-sweep, after which an odd cell's residual
 // is zero up to rounding (its x was just solved from its row), so only the
-// block's four even cells are summed.
-template <typename V>
+// block's four even cells are summed, one on each of its (J,K) lines.
+template <typename V, bool SKIP>
 __device__ __forceinline__ V block_residual(const MgLevelT<V> &F, int I, int J, int K)
 {
-    const Dims &fd = F.d;
+    Cell<V> e[4];
+    bool act[4];
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+        const int j0 = 2 * J - 2 + (c & 1), k0 = 2 * K - 2 + (c >> 1), i0 = 2 * I - 2 + ((j0 + k0) & 1);
+        const int i = min(i0, F.d.ni - 1), j = min(j0, F.d.nj - 1), k = min(k0, F.d.nk - 1);
+        e[c] = cell_at(F, (i - 1) >> 1, i, j, k, 0);
+        act[c] = i == i0 && j == j0 && k == k0 && F.act[e[c].n] != 0;
+    }
     V s = 0;
-    for (int c = 0; c < 8; c++) {
-        const int i = 2 * I - 2 + (c & 1), j = 2 * J - 2 + ((c >> 1) & 1), k = 2 * K - 2 + (c >> 2);
-        if (((i + j + k) & 1) != 0 || i > fd.ni - 1 || j > fd.nj - 1 || k > fd.nk - 1) continue;
-        const long long n = pos(F, i, j, k);
-        if (!F.act[n]) continue;
-        s += F.b[n] - F.ad[n] * F.x[n] - row_off(F, n, i, j, k);
+    if (SKIP && !(act[0] || act[1] || act[2] || act[3])) return s;
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+        const V r = F.b[e[c].n] - F.ad[e[c].n] * F.x[e[c].n] - row_off(F, e[c]);
+        if (act[c]) s += r;
     }
     return s;
 }
 
-template <typename V>
+template <typename V, bool SKIP>
 __global__ void __launch_bounds__(256) k_mg_restrict(MgLevelT<V> F, MgLevelT<V> C, int k0)
 {
     const int I = blockIdx.x * blockDim.x + threadIdx.x + 2;
     const int J = blockIdx.y * blockDim.y + threadIdx.y + 2;
     const int K = blockIdx.z + k0;
     if (I > C.d.ni - 1 || J > C.d.nj - 1 || K > C.d.nk - 1) return;
-    const V s = block_residual(F, I, J, K);
     const long long m = pos(C, I, J, K);
-    const V bc = C.act[m] ? s : (V)0;
+    const bool act = C.act[m] != 0;
+    const V ad = C.ad[m];
+    const V s = block_residual<V, SKIP>(F, I, J, K);
+    const V bc = act ? s : (V)0;
     C.b[m] = bc;
     // from x = 0 the even half of the first sweep is x = b/AD
-    C.x[m] = C.act[m] && ((I + J + K) & 1) == 0 ? bc / C.ad[m] : (V)0;
+    C.x[m] = act && ((I + J + K) & 1) == 0 ? bc / ad : (V)0;
 }
 
 // The coarse correction and the even half-sweep after it, in one pass.  The
@@ -229,15 +266,10 @@ __global__ void __launch_bounds__(256) k_mg_restrict(MgLevelT<V> F, MgLevelT<V> 
 // reads the odd neighbours only.  So each even cell reads its odd
 // neighbours' x plus their correction (what a separate correction pass would
 // have stored), and the odd cells, which the odd half-sweep that follows
-// solves from their rows in turn, are not corrected in memory.
-template <typename V>
-__device__ __forceinline__ V corrected(const MgLevelT<V> &F, const MgLevelT<V> &C, int i, int j, int k)
-{
-    const long long n = pos(F, i, j, k);
-    return F.act[n] ? F.x[n] + (V)MG_SCALE * C.x[pos(C, (i + 2) / 2, (j + 2) / 2, (k + 2) / 2)] : F.x[n];
-}
-
-template <typename V>
+// solves from their rows in turn, are not corrected in memory.  Of the six
+// neighbours one in each direction is in the cell's own block, so four coarse
+// values serve them.
+template <typename V, bool SKIP>
 __global__ void __launch_bounds__(256) k_mg_correct_even(MgLevelT<V> F, MgLevelT<V> C, int k0)
 {
     const int j = blockIdx.y * blockDim.y + threadIdx.y + 2;
@@ -246,12 +278,27 @@ __global__ void __launch_bounds__(256) k_mg_correct_even(MgLevelT<V> F, MgLevelT
     const int q = (int)(blockIdx.x * blockDim.x + threadIdx.x);
     const int i = 2 * q + 1 + ((1 + j + k) & 1);
     if (i < 2 || i > F.d.ni - 1) return;
-    const long long n = pos(F, i, j, k);
-    if (!F.act[n]) return;
-    const V off = F.ali[n] * corrected(F, C, i - 1, j, k) + F.aui[n] * corrected(F, C, i + 1, j, k)
-                + F.alj[n] * corrected(F, C, i, j - 1, k) + F.auj[n] * corrected(F, C, i, j + 1, k)
-                + F.alk[n] * corrected(F, C, i, j, k - 1) + F.auk[n] * corrected(F, C, i, j, k + 1);
-    F.x[n] = (F.b[n] - off) / F.ad[n];
+    const Cell<V> e = cell_at(F, q, i, j, k, 0);
+    const bool act = F.act[e.n] != 0;
+    if (SKIP && !act) return;
+    const int I = (i + 2) >> 1, J = (j + 2) >> 1, K = (k + 2) >> 1;
+    const bool oi = i & 1, oj = j & 1, ok = k & 1;   // the upper cell of its block
+    const V own = C.x[pos(C, I, J, K)];
+    const V xi = C.x[pos(C, oi ? I + 1 : I - 1, J, K)], xj = C.x[pos(C, I, oj ? J + 1 : J - 1, K)];
+    const V xk = C.x[pos(C, I, J, ok ? K + 1 : K - 1)];
+    const int lj = F.ld, lk = F.ld * F.d.nj;
+    const int n6[6] = {e.o - 1 + e.p, e.o + e.p, e.o - lj, e.o + lj, e.o - lk, e.o + lk};
+    const V c6[6] = {oi ? own : xi, oi ? xi : own, oj ? own : xj, oj ? xj : own, ok ? own : xk, ok ? xk : own};
+    V y[6];
+#pragma unroll
+    for (int a = 0; a < 6; a++) {
+        const V x = F.x[n6[a]];
+        y[a] = F.act[n6[a]] ? x + (V)MG_SCALE * c6[a] : x;
+    }
+    const V off = F.ali[e.n] * y[0] + F.aui[e.n] * y[1] + F.alj[e.n] * y[2] + F.auj[e.n] * y[3]
+                + F.alk[e.n] * y[4] + F.auk[e.n] * y[5];
+    const V x = (F.b[e.n] - off) / F.ad[e.n];
+    if (act) F.x[e.n] = x;
 }
 
 // level-0 right-hand side from a vector of the grid (natural order) on the K
@@ -307,7 +354,7 @@ __global__ void __launch_bounds__(256) k_mg_out_resid(const MgLevelT<V> L, T *__
             continue;
         }
         const V xm = L.x[m];
-        const V rv = L.b[m] - L.ad[m] * xm - row_off(L, m, i, j, k);
+        const V rv = L.b[m] - L.ad[m] * xm - row_off(L, cell_at(L, (i - 1) >> 1, i, j, k, (i + j + k) & 1));
         x[n] = (T)xm;
         r[n] = (T)rv;
         a += (double)rv * (double)rv;
@@ -329,121 +376,243 @@ __global__ void __launch_bounds__(256) k_mg_out_resid(const MgLevelT<V> L, T *__
     }
 }
 
-// The V-cycle below level t0 inside one workgroup: for each level down to the
-// coarsest the odd half-sweep (the even half was set with b), the coarse
-// right-hand side; MG_COARSE sweeps on the coarsest; then up: the even
-// half-sweep with the correction, and the odd one.  The coarsest level, whose
-// sweeps are most of the tail's phases, is swept in LDS: its x and b are
-// copied in, each thread keeps its cell's row in registers, and x goes back
-// at the end, so those phases touch no memory.  Levels are a kernel argument
-// (at most CAD_MG_MAX).
-constexpr int TAIL_THREADS = 1024;
-constexpr int TAIL_LDS_CELLS = 8192;         // positions of the coarsest level held in LDS
+// The V-cycle below level t0 inside one workgroup (k_mg_tail): for each level
+// down to the coarsest the odd half-sweep (the even half is set with b) and the
+// coarse right-hand side; MG_COARSE sweeps on the coarsest; then up: the
+// correction, the even half-sweep and the odd one.  Its time is the latency of
+// some forty phases, so nothing in them touches memory: x is in LDS (natural
+// order with a ghost layer), and each thread keeps its cells' rows and b in
+// registers, loaded at once at the start.  On 32x16x8 cells and three levels
+// below them this takes 17 us where phases that read the rows from memory took
+// 34, on 64x4x12 and one below 13 against 25.
+//
+// A thread owns up to A cells of each colour on level t0 and, below it, two,
+// one and one (a coarsened level has at most 27/125 of the cells).  The
+// residuals of every level have their own zeroed place in LDS, so a block that
+// reaches beyond the grid sums its ghost cells' zeros.
+constexpr int TAIL_THREADS = 512;
+constexpr int TAIL_LEVELS = 4;
+constexpr int TAIL_LDS = 18432;              // values of x and residuals
 
 template <typename V>
 struct MgTail {
-    MgLevelT<V> L[CAD_MG_MAX];
+    MgLevelT<V> L[TAIL_LEVELS];
+    float inv_h[TAIL_LEVELS], inv_j[TAIL_LEVELS];   // 1 / positions a half line, 1 / lines a plane
+    int base[TAIL_LEVELS];                   // first LDS position of a level's x
+    int res, nt;                             // residuals are res behind x; number of levels
 };
 
 template <typename V>
-__device__ void tail_half(const MgLevelT<V> &L, int color)
+struct TailRow {
+    V ad, li, ui, lj, uj, lk, uk, b;
+    int o, n;                                // LDS position and position in the level; o < 0: no cell
+    int up, src;                             // LDS positions of its coarse cell's x and of its block's first residual
+    bool act;
+};
+
+// positions of a colour on the interior part of a half line
+__device__ __host__ __forceinline__ int tail_half(int ni) { return (ni - 1) / 2; }
+
+template <typename V>
+__device__ __forceinline__ void tail_load(const MgTail<V> &T, int l, int color, int e, TailRow<V> &r)
 {
-    const int ni = L.d.ni - 2, nj = L.d.nj - 2, nk = L.d.nk - 2;
-    const int cells = ni * nj * nk;
-    for (int q = threadIdx.x; q < cells; q += blockDim.x) {
-        const int i = q % ni + 2, j = (q / ni) % nj + 2, k = q / (ni * nj) + 2;
-        if (((i + j + k) & 1) != color) continue;
-        const long long n = pos(L, i, j, k);
-        if (L.act[n]) L.x[n] = (L.b[n] - row_off(L, n, i, j, k)) / L.ad[n];
+    const MgLevelT<V> &L = T.L[l];
+    const int ni = L.d.ni, nj = L.d.nj, nk = L.d.nk;
+    // e / h: (e + 1/2) / h is at least 1/2h from a whole number, far beyond the product's rounding
+    const int line = (int)(((float)e + 0.5f) * T.inv_h[l]), u = e - line * tail_half(ni);
+    const int kk = (int)(((float)line + 0.5f) * T.inv_j[l]), k = kk + 2, j = line - kk * (nj - 2) + 2;
+    const int i = 2 * u + 2 + ((color + j + k) & 1);
+    const bool in = k <= nk - 1 && i <= ni - 1;
+    r.n = in ? (int)pos(L, i, j, k) : 0;
+    r.o = in ? T.base[l] + i - 1 + ni * (j - 1 + nj * (k - 1)) : -1;
+    r.act = in && L.act[r.n] != 0;
+    if (l + 1 < T.nt) {
+        const Dims &c = T.L[l + 1].d;
+        r.up = T.base[l + 1] + ((i + 2) >> 1) - 1 + c.ni * (((j + 2) >> 1) - 1 + c.nj * (((k + 2) >> 1) - 1));
+    }
+    if (l > 0) {
+        const Dims &f = T.L[l - 1].d;
+        r.src = T.res + T.base[l - 1] + 2 * i - 3 + f.ni * (2 * j - 3 + f.nj * (2 * k - 3));
+    }
+    r.ad = L.ad[r.n];
+    r.li = L.ali[r.n];
+    r.ui = L.aui[r.n];
+    r.lj = L.alj[r.n];
+    r.uj = L.auj[r.n];
+    r.lk = L.alk[r.n];
+    r.uk = L.auk[r.n];
+    r.b = l == 0 ? L.b[r.n] : (V)0;
+}
+
+template <typename V>
+__device__ __forceinline__ V tail_off(const TailRow<V> &r, const V *x, int ni, int nij)
+{
+    const int o = r.o;
+    return r.li * x[o - 1] + r.ui * x[o + 1] + r.lj * x[o - ni] + r.uj * x[o + ni] + r.lk * x[o - nij]
+         + r.uk * x[o + nij];
+}
+
+template <typename V, int N>
+__device__ __forceinline__ void tail_sweep(const TailRow<V> (&r)[N], V *x, int ni, int nij)
+{
+#pragma unroll
+    for (int s = 0; s < N; s++)
+        if (r[s].act) x[r[s].o] = (r[s].b - tail_off(r[s], x, ni, nij)) / r[s].ad;
+}
+
+// Down from a level with N rows of each colour a thread to one with M.
+template <typename V, int N, int M>
+__device__ __forceinline__ void tail_down(const MgTail<V> &T, int l, const TailRow<V> (&ev)[N], const TailRow<V> (&od)[N],
+                                          TailRow<V> (&cev)[M], TailRow<V> (&cod)[M], V *x)
+{
+    const int ni = T.L[l].d.ni, nij = ni * T.L[l].d.nj;
+    tail_sweep(od, x, ni, nij);
+    __syncthreads();
+#pragma unroll
+    for (int s = 0; s < N; s++)
+        if (ev[s].act) x[T.res + ev[s].o] = ev[s].b - ev[s].ad * x[ev[s].o] - tail_off(ev[s], x, ni, nij);
+    __syncthreads();
+    // the block's even cells in the order of k_mg_restrict
+    auto sum = [&](const TailRow<V> &r) {
+        const V *q = x + r.src;
+        return q[0] + q[1 + ni] + q[1 + nij] + q[ni + nij];
+    };
+#pragma unroll
+    for (int s = 0; s < M; s++) {
+        if (cev[s].act) {
+            cev[s].b = sum(cev[s]);
+            x[cev[s].o] = cev[s].b / cev[s].ad;   // the even half from x = 0
+        }
+        if (cod[s].act) cod[s].b = sum(cod[s]);
     }
     __syncthreads();
 }
 
-// the even half-sweep of F with the correction from C (k_mg_correct_even)
-template <typename V>
-__device__ void tail_correct_even(const MgLevelT<V> &F, const MgLevelT<V> &C)
+// MG_COARSE sweeps of the coarsest level (the even half of the first came with
+// b).  A level whose colours fit the first wave is swept by it alone.
+template <typename V, int N>
+__device__ __forceinline__ void tail_coarsest(const MgTail<V> &T, int l, const TailRow<V> (&ev)[N],
+                                              const TailRow<V> (&od)[N], V *x)
 {
-    const int ni = F.d.ni - 2, nj = F.d.nj - 2, nk = F.d.nk - 2;
-    for (int q = threadIdx.x; q < ni * nj * nk; q += blockDim.x) {
-        const int i = q % ni + 2, j = (q / ni) % nj + 2, k = q / (ni * nj) + 2;
-        if (((i + j + k) & 1) != 0) continue;
-        const long long n = pos(F, i, j, k);
-        if (!F.act[n]) continue;
-        const V off = F.ali[n] * corrected(F, C, i - 1, j, k) + F.aui[n] * corrected(F, C, i + 1, j, k)
-                    + F.alj[n] * corrected(F, C, i, j - 1, k) + F.auj[n] * corrected(F, C, i, j + 1, k)
-                    + F.alk[n] * corrected(F, C, i, j, k - 1) + F.auk[n] * corrected(F, C, i, j, k + 1);
-        F.x[n] = (F.b[n] - off) / F.ad[n];
-    }
-    __syncthreads();
-}
-
-// MG_COARSE sweeps of the coarsest level B in LDS (the even half of the
-// first came with b); at most TAIL_THREADS cells and TAIL_LDS_CELLS
-// positions (the host sweeps larger coarsest levels in memory)
-template <typename V>
-__device__ void tail_coarsest(const MgLevelT<V> &B)
-{
-    __shared__ V xs[TAIL_LDS_CELLS], bs[TAIL_LDS_CELLS];
-    const int ns = B.ld * B.d.nj * B.d.nk;
-    for (int p = threadIdx.x; p < ns; p += blockDim.x) {
-        xs[p] = B.x[p];
-        bs[p] = B.b[p];
-    }
-    const int ni = B.d.ni - 2, nj = B.d.nj - 2, nk = B.d.nk - 2;
-    const int q = threadIdx.x;
-    const bool on = q < ni * nj * nk;
-    const int i = on ? q % ni + 2 : 2, j = on ? (q / ni) % nj + 2 : 2, k = on ? q / (ni * nj) + 2 : 2;
-    const long long n = pos(B, i, j, k);
-    const bool act = on && B.act[n];
-    const bool odd = ((i + j + k) & 1) != 0;
-    const V ad = act ? B.ad[n] : (V)1, li = act ? B.ali[n] : (V)0, ui = act ? B.aui[n] : (V)0;
-    const V lj = act ? B.alj[n] : (V)0, uj = act ? B.auj[n] : (V)0, lk = act ? B.alk[n] : (V)0;
-    const V uk = act ? B.auk[n] : (V)0;
-    const long long pi0 = pos(B, i - 1, j, k), pi1 = pos(B, i + 1, j, k), pj0 = pos(B, i, j - 1, k);
-    const long long pj1 = pos(B, i, j + 1, k), pk0 = pos(B, i, j, k - 1), pk1 = pos(B, i, j, k + 1);
-    __syncthreads();
-    for (int h = 1; h < 2 * MG_COARSE; h++) {
-        // h odd: the odd half, h even: the even half
-        if (act && odd == ((h & 1) != 0))
-            xs[n] = (bs[n] - (li * xs[pi0] + ui * xs[pi1] + lj * xs[pj0] + uj * xs[pj1] + lk * xs[pk0]
-                              + uk * xs[pk1])) / ad;
-        __syncthreads();
-    }
-    if (on) B.x[n] = xs[n];
-    __syncthreads();
-}
-
-template <typename V>
-__global__ void __launch_bounds__(TAIL_THREADS) k_mg_tail(MgTail<V> T, int t0, int nl, int lds_coarsest)
-{
-    for (int l = t0; l < nl - 1; l++) {
-        const MgLevelT<V> &F = T.L[l], &C = T.L[l + 1];
-        tail_half(F, 1);
-        const int ni = C.d.ni - 2, nj = C.d.nj - 2, nk = C.d.nk - 2;
-        for (int q = threadIdx.x; q < ni * nj * nk; q += blockDim.x) {
-            const int I = q % ni + 2, J = (q / ni) % nj + 2, K = q / (ni * nj) + 2;
-            const V s = block_residual(F, I, J, K);
-            const long long m = pos(C, I, J, K);
-            const V bc = C.act[m] ? s : (V)0;
-            C.b[m] = bc;
-            C.x[m] = C.act[m] && ((I + J + K) & 1) == 0 ? bc / C.ad[m] : (V)0;
+    const Dims &d = T.L[l].d;
+    const int ni = d.ni, nij = d.ni * d.nj;
+    if (tail_half(ni) * (d.nj - 2) * (d.nk - 2) <= 64) {
+        if (threadIdx.x < 64) {
+            for (int s = 0; s < MG_COARSE; s++) {
+                if (s) tail_sweep(ev, x, ni, nij);
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+                tail_sweep(od, x, ni, nij);
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+            }
         }
         __syncthreads();
+        return;
     }
-    const MgLevelT<V> &B = T.L[nl - 1];
-    if (lds_coarsest) {
-        tail_coarsest(B);
+    for (int s = 0; s < MG_COARSE; s++) {
+        if (s) {
+            tail_sweep(ev, x, ni, nij);
+            __syncthreads();
+        }
+        tail_sweep(od, x, ni, nij);
+        __syncthreads();
+    }
+}
+
+template <typename V, int N>
+__device__ __forceinline__ void tail_up(const MgTail<V> &T, int l, const TailRow<V> (&ev)[N], const TailRow<V> (&od)[N],
+                                        V *x)
+{
+    const int ni = T.L[l].d.ni, nij = ni * T.L[l].d.nj;
+#pragma unroll
+    for (int s = 0; s < N; s++)
+        if (od[s].act) x[od[s].o] = x[od[s].o] + (V)MG_SCALE * x[od[s].up];
+    __syncthreads();
+    tail_sweep(ev, x, ni, nij);
+    __syncthreads();
+    tail_sweep(od, x, ni, nij);
+    __syncthreads();
+}
+
+template <typename V, int A>
+__global__ void __launch_bounds__(TAIL_THREADS) k_mg_tail(MgTail<V> T)
+{
+    __shared__ V x[TAIL_LDS];
+    TailRow<V> e0[A], o0[A], e1[2], o1[2], e2[1], o2[1], e3[1], o3[1];
+    const int t = threadIdx.x;
+#pragma unroll
+    for (int s = 0; s < A; s++) {
+        tail_load(T, 0, 0, t + s * TAIL_THREADS, e0[s]);
+        tail_load(T, 0, 1, t + s * TAIL_THREADS, o0[s]);
+    }
+    if (T.nt > 1) {
+#pragma unroll
+        for (int s = 0; s < 2; s++) {
+            tail_load(T, 1, 0, t + s * TAIL_THREADS, e1[s]);
+            tail_load(T, 1, 1, t + s * TAIL_THREADS, o1[s]);
+        }
+    }
+    if (T.nt > 2) {
+        tail_load(T, 2, 0, t, e2[0]);
+        tail_load(T, 2, 1, t, o2[0]);
+    }
+    if (T.nt > 3) {
+        tail_load(T, 3, 0, t, e3[0]);
+        tail_load(T, 3, 1, t, o3[0]);
+    }
+    for (int p = t; p < 2 * T.res; p += TAIL_THREADS) x[p] = (V)0;
+    __syncthreads();
+    // from x = 0 the even half of the first sweep is x = b/AD
+#pragma unroll
+    for (int s = 0; s < A; s++)
+        if (e0[s].act) x[e0[s].o] = e0[s].b / e0[s].ad;
+    __syncthreads();
+    if (T.nt > 1) {
+        tail_down(T, 0, e0, o0, e1, o1, x);
+        if (T.nt > 2) {
+            tail_down(T, 1, e1, o1, e2, o2, x);
+            if (T.nt > 3) {
+                tail_down(T, 2, e2, o2, e3, o3, x);
+                tail_coarsest(T, 3, e3, o3, x);
+                tail_up(T, 2, e2, o2, x);
+            } else {
+                tail_coarsest(T, 2, e2, o2, x);
+            }
+            tail_up(T, 1, e1, o1, x);
+        } else {
+            tail_coarsest(T, 1, e1, o1, x);
+        }
+        tail_up(T, 0, e0, o0, x);
     } else {
-        tail_half(B, 1);
-        for (int s = 1; s < MG_COARSE; s++) {
-            tail_half(B, 0);
-            tail_half(B, 1);
-        }
+        tail_coarsest(T, 0, e0, o0, x);
     }
-    for (int l = nl - 2; l >= t0; l--) {
-        tail_correct_even(T.L[l], T.L[l + 1]);
-        tail_half(T.L[l], 1);
+#pragma unroll
+    for (int s = 0; s < A; s++) {
+        if (e0[s].o >= 0) T.L[0].x[e0[s].n] = x[e0[s].o];
+        if (o0[s].o >= 0) T.L[0].x[o0[s].n] = x[o0[s].o];
     }
+}
+
+// The tail from level t0 on: the rows a thread of k_mg_tail holds of each colour
+// on level t0, or 0 where the levels do not fit it.
+template <typename V>
+int tail_rows(const MgLevelT<V> *mg, int nl, int t0, MgTail<V> *T)
+{
+    if (nl - t0 > TAIL_LEVELS) return 0;
+    long long lds = 0, need[TAIL_LEVELS] = {0, 0, 0, 0};
+    for (int l = t0; l < nl; l++) {
+        const Dims &d = mg[l].d;
+        const int h = tail_half(d.ni), q = l - t0;
+        need[q] = ((long long)h * (d.nj - 2) * (d.nk - 2) + TAIL_THREADS - 1) / TAIL_THREADS;
+        T->L[q] = mg[l];
+        T->inv_h[q] = 1.0f / (float)h;
+        T->inv_j[q] = 1.0f / (float)(d.nj - 2);
+        T->base[q] = (int)std::min(lds, (long long)TAIL_LDS);
+        lds += d.nc;
+    }
+    T->res = (int)std::min(lds, (long long)TAIL_LDS);
+    T->nt = nl - t0;
+    if (2 * lds > TAIL_LDS || need[0] > 6 || need[1] > 2 || need[2] > 1 || need[3] > 1) return 0;
+    return need[0] <= 2 ? 2 : need[0] <= 4 ? 4 : 6;
 }
 
 dim3 lvl_grid(const Dims &d, int k0, int k1)
@@ -458,13 +627,15 @@ dim3 half_grid(const Dims &d, int k0, int k1)
     return dim3((unsigned)((half + 63) / 64), (unsigned)((d.nj - 2 + 3) / 4), (unsigned)(k1 - k0 + 1));
 }
 
-// half-sweeps of colours c0..1 on K planes k0..k1
+// half-sweep of a colour on K planes k0..k1
 template <typename V>
-int smooth(cad_ctx *c, const MgLevelT<V> &L, int k0, int k1, int c0)
+int smooth(cad_ctx *c, const MgLevelT<V> &L, int k0, int k1, int color)
 {
     const dim3 b(64, 4, 1), g = half_grid(L.d, k0, k1);
-    for (int color = c0; color <= 1; color++)
-        hipLaunchKernelGGL(k_mg_smooth<V>, g, b, 0, c->stream, L, color, k0);
+    if (L.d.nc > MG_SKIP_CELLS)
+        hipLaunchKernelGGL((k_mg_smooth<V, true>), g, b, 0, c->stream, L, color, k0);
+    else
+        hipLaunchKernelGGL((k_mg_smooth<V, false>), g, b, 0, c->stream, L, color, k0);
     CAD_CHECK(hipGetLastError());
     return CAD_OK;
 }
@@ -574,11 +745,11 @@ int vcycle(cad_ctx *c, const MgLevelT<V> *mg, int nl, const T *y, T *x, int k0, 
     const dim3 b(64, 4, 1);
     hipLaunchKernelGGL((k_mg_in<V, T>), lvl_grid(mg[0].d, k0, k1), b, 0, c->stream, mg[0], y, k0);
     CAD_CHECK(hipGetLastError());
-    // the first level small enough for one workgroup
-    int t0 = nl - 1;
-    while (t0 > 0 && (long long)(mg[t0 - 1].d.ni - 2) * (mg[t0 - 1].d.nj - 2) * (mg[t0 - 1].d.nk - 2) <=
-                         MG_TAIL_CELLS)
-        t0--;
+    // the first level from which on one workgroup holds the rest (nl: none, the
+    // coarsest is too large for it)
+    MgTail<V> tl;
+    int t0 = 0, rows = 0;
+    while (t0 < nl && !(rows = tail_rows(mg, nl, t0, &tl))) t0++;
     // Each level's passes run on the K planes that can hold its active rows:
     // level 0's k0..k1, and on a coarser level the planes of their parents
     // (fine plane k lies in coarse plane (k + 2) / 2).  Rows outside are
@@ -592,24 +763,37 @@ int vcycle(cad_ctx *c, const MgLevelT<V> *mg, int nl, const T *y, T *x, int k0, 
         hi[l] = std::min(mg[l].d.nk - 1, (hi[l - 1] + 2) / 2);
     }
     // down: the odd half-sweep (the even half came with b), the coarse b
-    for (int l = 0; l < t0; l++) {
+    for (int l = 0; l < std::min(t0, nl - 1); l++) {
         const MgLevelT<V> &F = mg[l], &C = mg[l + 1];
         RET_IF(smooth(c, F, lo[l], hi[l], 1));
-        hipLaunchKernelGGL(k_mg_restrict<V>, lvl_grid(C.d, lo[l + 1], hi[l + 1]), b, 0, c->stream, F, C,
-                           lo[l + 1]);
+        const dim3 g = lvl_grid(C.d, lo[l + 1], hi[l + 1]);
+        if (F.d.nc > MG_SKIP_CELLS)
+            hipLaunchKernelGGL((k_mg_restrict<V, true>), g, b, 0, c->stream, F, C, lo[l + 1]);
+        else
+            hipLaunchKernelGGL((k_mg_restrict<V, false>), g, b, 0, c->stream, F, C, lo[l + 1]);
         CAD_CHECK(hipGetLastError());
     }
-    MgTail<V> tl;
-    for (int l = 0; l < nl; l++) tl.L[l] = mg[l];
-    const MgLevelT<V> &top = mg[nl - 1];
-    const int lds = (long long)(top.d.ni - 2) * (top.d.nj - 2) * (top.d.nk - 2) <= TAIL_THREADS &&
-                    (long long)top.ld * top.d.nj * top.d.nk <= TAIL_LDS_CELLS;
-    hipLaunchKernelGGL(k_mg_tail<V>, dim3(1), dim3(TAIL_THREADS), 0, c->stream, tl, t0, nl, lds);
-    CAD_CHECK(hipGetLastError());
+    if (t0 == nl) {
+        const MgLevelT<V> &B = mg[nl - 1];
+        for (int h = 1; h < 2 * MG_COARSE; h++) RET_IF(smooth(c, B, lo[nl - 1], hi[nl - 1], h & 1));
+    } else {
+        const dim3 tb(TAIL_THREADS);
+        if (rows == 2)
+            hipLaunchKernelGGL((k_mg_tail<V, 2>), dim3(1), tb, 0, c->stream, tl);
+        else if (rows == 4)
+            hipLaunchKernelGGL((k_mg_tail<V, 4>), dim3(1), tb, 0, c->stream, tl);
+        else
+            hipLaunchKernelGGL((k_mg_tail<V, 6>), dim3(1), tb, 0, c->stream, tl);
+        CAD_CHECK(hipGetLastError());
+    }
     // up: correct, then one sweep (the correction rides on the even half)
-    for (int l = t0 - 1; l >= 0; l--) {
+    for (int l = std::min(t0, nl - 1) - 1; l >= 0; l--) {
         const MgLevelT<V> &F = mg[l], &C = mg[l + 1];
-        hipLaunchKernelGGL(k_mg_correct_even<V>, half_grid(F.d, lo[l], hi[l]), b, 0, c->stream, F, C, lo[l]);
+        const dim3 g = half_grid(F.d, lo[l], hi[l]);
+        if (F.d.nc > MG_SKIP_CELLS)
+            hipLaunchKernelGGL((k_mg_correct_even<V, true>), g, b, 0, c->stream, F, C, lo[l]);
+        else
+            hipLaunchKernelGGL((k_mg_correct_even<V, false>), g, b, 0, c->stream, F, C, lo[l]);
         CAD_CHECK(hipGetLastError());
         RET_IF(smooth(c, F, lo[l], hi[l], 1));
     }
