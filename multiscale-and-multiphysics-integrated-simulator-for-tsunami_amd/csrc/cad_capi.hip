@@ -236,6 +236,7 @@ void cad_destroy(cad_ctx *c)
     cad_tdoor_free(c);
     cad_wave_free(c);
     cad_wave_theory_free(c);
+    cad_mixed_free(c);
     cad_mg_free(c);
     cad_learned_free(c);
     cad_kt_free(c);

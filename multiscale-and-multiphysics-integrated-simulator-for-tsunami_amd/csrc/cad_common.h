@@ -126,7 +126,7 @@ inline dim3 cell_grid(const Dims &d)
 constexpr int REDUCE_BLOCKS = 1024;
 constexpr int REDUCE_THREADS = 256;
 constexpr int REDUCE_SLOTS = 6;   // products whose partials are kept apart
-constexpr int CAD_REC = 8;        // first double of the solve's record in host_red
+constexpr int CAD_REC = 8;        // first double of the solves' records in host_red
 
 // One level of the multigrid (cad_mg.hip): a grid with one ghost layer, its
 // 7-point rows (inactive rows AD = 1, no couplings), the level's unknowns and
@@ -141,8 +141,6 @@ struct MgLevelT {
     V *ad, *ali, *alj, *alk, *aui, *auj, *auk;
     V *x, *b;
     unsigned char *act;
-    V *nad, *nali, *nalj, *nalk, *naui, *nauj, *nauk;
-    unsigned char *nact;
 };
 typedef MgLevelT<float> MgLevel;
 
@@ -262,6 +260,7 @@ struct cad_ctx {
     int mg64_n;
     unsigned long long mg_span;   // cells in the active index range of the current solve
     int mg_k0, mg_k1;             // K planes of level 0's passes in the current solve
+    struct cad_mixed *mx;         // the mixed form's vectors and captured iteration (cad_refine.hip)
     int mg_set_k0, mg_set_k1;     // K planes level 0's rows were last built on (0: none yet)
     // the learned form's network, Krylov basis and counters (cad_learned.hip),
     // allocated when its weights are set
@@ -340,7 +339,11 @@ int cad_mg_alloc(cad_ctx *c);
 void cad_mg_free(cad_ctx *c);
 int cad_mg_setup(cad_ctx *c);
 int cad_mg_apply(cad_ctx *c, const double *y, double *x, int k0, int k1);
-int cad_mg_apply32(cad_ctx *c, const float *y, float *x, int k0, int k1);
+// one V-cycle in FP32 with level 0's right-hand side b and result x in its
+// layout, x holding the first half-sweep's even cells (b/AD) and 0 on inactive ones
+int cad_mg_cycle(cad_ctx *c, float *b, float *x);
+void cad_mixed_free(cad_ctx *c);
+int cad_wait_record(cad_ctx *c, int at, double tag, double *out);
 // cad_mg_apply and r = y - A x on the V-cycle's FP32 level-0 matrix, with the
 // block partials of sum r^2 and of the row count at part[b * stride] and
 // part[b * stride + 1], b < REDUCE_BLOCKS

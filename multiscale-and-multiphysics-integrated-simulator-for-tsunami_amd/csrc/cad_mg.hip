@@ -21,13 +21,12 @@
 // positive, is inactive.
 //
 // Storage.  Each level stores the two colours of the red-black ordering
-// apart: a (J,K) line of ld cells (NUMI rounded up to even) holds first its
+// apart: a (J,K) line of ld cells (NUMI rounded up to a multiple of eight) holds first its
 // cells with I+J+K even, then those with I+J+K odd, each half in ascending
 // I.  A half-sweep then reads and writes whole lines of its own colour and
 // reads the other colour's x at the same positions of the neighbouring lines,
 // so a thread's neighbours are its neighbour threads' cells and no line is
-// fetched for half of its cells.  Level 0 also keeps its rows in the grid's
-// natural order (for the FP32 matvec of cad_refine.hip).
+// fetched for half of its cells.
 //
 // V-cycle.  Red-black Gauss-Seidel (one sweep = the cells with I+J+K even,
 // then odd) before and after the coarse correction; the residual of the fine
@@ -69,8 +68,7 @@ __device__ __forceinline__ long long nat(const Dims &d, int i, int j, int k)
     return (long long)(i - 1) + (long long)d.ni * (j - 1) + d.nij * (k - 1);
 }
 
-// level 0 from the FP64 matrix: the colour-split rows and, where the level
-// has them, the natural-order copy
+// level 0 from the FP64 matrix
 template <typename V>
 __global__ void __launch_bounds__(256) k_mg_fine(Dims d, const double *__restrict__ ad,
                                                  const double *__restrict__ ali,
@@ -97,16 +95,6 @@ __global__ void __launch_bounds__(256) k_mg_fine(Dims d, const double *__restric
     L.aui[m] = r[4];
     L.auj[m] = r[5];
     L.auk[m] = r[6];
-    if (L.nad) {
-        L.nact[n] = a ? 1 : 0;
-        L.nad[n] = r[0];
-        L.nali[n] = r[1];
-        L.nalj[n] = r[2];
-        L.nalk[n] = r[3];
-        L.naui[n] = r[4];
-        L.nauj[n] = r[5];
-        L.nauk[n] = r[6];
-    }
 }
 
 // Galerkin coarse row of coarse interior cell (I,J,K), K from k0; one thread
@@ -645,7 +633,7 @@ void free_levels(MgLevelT<V> *mg, int &n)
 {
     for (int l = 0; l < n; l++) {
         MgLevelT<V> &L = mg[l];
-        void *p[] = {L.ad, L.ali, L.alj, L.alk, L.aui, L.auj, L.auk, L.x, L.b, L.act, L.nad, L.nact};
+        void *p[] = {L.ad, L.ali, L.alj, L.alk, L.aui, L.auj, L.auk, L.x, L.b, L.act};
         for (void *q : p)
             if (q) (void)hipFree(q);
         L = MgLevelT<V>();
@@ -653,11 +641,10 @@ void free_levels(MgLevelT<V> *mg, int &n)
     n = 0;
 }
 
-// The levels of a grid: colour-split arrays of ld x NUMJ x NUMK per level
-// (and level 0's natural-order copy when natural is set), each level counted
+// The levels of a grid: colour-split arrays of ld x NUMJ x NUMK per level, each level counted
 // before its arrays so that a failed allocation frees what was allocated.
 template <typename V>
-int alloc_levels(const Dims &d0, MgLevelT<V> *mg, int &nl, bool natural)
+int alloc_levels(const Dims &d0, MgLevelT<V> *mg, int &nl)
 {
     if (nl > 0) return CAD_OK;
     Dims d = d0;
@@ -667,7 +654,7 @@ int alloc_levels(const Dims &d0, MgLevelT<V> *mg, int &nl, bool natural)
         MgLevelT<V> &L = mg[n];
         L = MgLevelT<V>();
         L.d = d;
-        L.ld = (d.ni + 1) / 2 * 2;
+        L.ld = (d.ni + 7) / 8 * 8;   // half lines of whole 16-byte vectors
         nl = n + 1;
         const size_t ns = (size_t)L.ld * d.nj * d.nk;
         V **f[] = {&L.ad, &L.ali, &L.alj, &L.alk, &L.aui, &L.auj, &L.auk, &L.x, &L.b};
@@ -677,19 +664,6 @@ int alloc_levels(const Dims &d0, MgLevelT<V> *mg, int &nl, bool natural)
         }
         CAD_CHECK(hipMalloc((void **)&L.act, ns));
         CAD_CHECK(hipMemset(L.act, 0, ns));
-        if (n == 0 && natural) {
-            const size_t nc = (size_t)d.nc;
-            CAD_CHECK(hipMalloc((void **)&L.nad, 7 * nc * sizeof(V)));
-            CAD_CHECK(hipMalloc((void **)&L.nact, nc));
-            CAD_CHECK(hipMemset(L.nad, 0, 7 * nc * sizeof(V)));
-            CAD_CHECK(hipMemset(L.nact, 0, nc));
-            L.nali = L.nad + nc;
-            L.nalj = L.nali + nc;
-            L.nalk = L.nalj + nc;
-            L.naui = L.nalk + nc;
-            L.nauj = L.naui + nc;
-            L.nauk = L.nauj + nc;
-        }
         n++;
         // coarsen while every interior extent is at least 4
         const int ei = d.ni - 2, ej = d.nj - 2, ek = d.nk - 2;
@@ -735,16 +709,12 @@ int setup_levels(cad_ctx *c, MgLevelT<V> *mg, int nl, int lo, int hi)
     return CAD_OK;
 }
 
-// x = M^-1 y: one V-cycle from x = 0; k0..k1 limits level 0 to the K planes
-// that hold active cells.  With r set, also r = y - A x on level 0's matrix
-// and the partials of its sum of squares (k_mg_out_resid, REDUCE_BLOCKS blocks).
-template <typename V, typename T>
-int vcycle(cad_ctx *c, const MgLevelT<V> *mg, int nl, const T *y, T *x, int k0, int k1, T *r = nullptr,
-           double *part = nullptr, int stride = 0)
+// One V-cycle's passes; level 0 holds b and the first half-sweep's x.  k0..k1
+// limits level 0 to the K planes that hold active cells.
+template <typename V>
+int passes(cad_ctx *c, const MgLevelT<V> *mg, int nl, int k0, int k1)
 {
     const dim3 b(64, 4, 1);
-    hipLaunchKernelGGL((k_mg_in<V, T>), lvl_grid(mg[0].d, k0, k1), b, 0, c->stream, mg[0], y, k0);
-    CAD_CHECK(hipGetLastError());
     // the first level from which on one workgroup holds the rest (nl: none, the
     // coarsest is too large for it)
     MgTail<V> tl;
@@ -797,6 +767,19 @@ int vcycle(cad_ctx *c, const MgLevelT<V> *mg, int nl, const T *y, T *x, int k0, 
         CAD_CHECK(hipGetLastError());
         RET_IF(smooth(c, F, lo[l], hi[l], 1));
     }
+    return CAD_OK;
+}
+
+// x = M^-1 y: one V-cycle from x = 0.  With r set, also r = y - A x on level 0's matrix
+// and the partials of its sum of squares (k_mg_out_resid, REDUCE_BLOCKS blocks).
+template <typename V, typename T>
+int vcycle(cad_ctx *c, const MgLevelT<V> *mg, int nl, const T *y, T *x, int k0, int k1, T *r = nullptr,
+           double *part = nullptr, int stride = 0)
+{
+    const dim3 b(64, 4, 1);
+    hipLaunchKernelGGL((k_mg_in<V, T>), lvl_grid(mg[0].d, k0, k1), b, 0, c->stream, mg[0], y, k0);
+    CAD_CHECK(hipGetLastError());
+    RET_IF(passes(c, mg, nl, k0, k1));
     if (r)
         hipLaunchKernelGGL((k_mg_out_resid<V, T>), dim3(REDUCE_BLOCKS), dim3(256), 0, c->stream, mg[0], x, r, k0, k1,
                            part, stride);
@@ -812,9 +795,7 @@ int vcycle(cad_ctx *c, const MgLevelT<V> *mg, int nl, const T *y, T *x, int k0, 
 // neighbours read once: 10 values + 1 byte per cell and colour pair), the
 // residual-restriction of the even cells (7 coefficients, b, x, activity,
 // and a share of the coarse b and x) and the coarse x that the corrected
-// even half-sweep reads; on the coarsest level MG_COARSE full sweeps; per cell of level
-// 0's K range the FP64 input read with b and x written (AD and the activity
-// read), and x and the activity read with the FP64 output written.
+// even half-sweep reads; on the coarsest level MG_COARSE full sweeps.
 double vcycle_bytes(const cad_ctx *c, const Dims *dims, int nl, int vs)
 {
     const double half = (10.0 * vs + 1.0) / 2.0;
@@ -825,7 +806,6 @@ double vcycle_bytes(const cad_ctx *c, const Dims *dims, int nl, int vs)
         const Dims &d = dims[l];
         const int planes = l == 0 ? c->mg_k1 - c->mg_k0 + 1 : d.nk - 2;
         const double cells = (double)(d.ni - 2) * (double)(d.nj - 2) * (double)planes;
-        if (l == 0) by += ((8.0 + 3.0 * vs + 1.0) + (vs + 8.0 + 1.0)) * cells;
         by += l == nl - 1 ? 2.0 * half * MG_COARSE * cells : (3.0 * half + restr + prol) * cells;
     }
     return by;
@@ -840,7 +820,7 @@ void cad_mg_free(cad_ctx *c)
     free_levels(c->mg64, c->mg64_n);
 }
 
-int cad_mg_alloc(cad_ctx *c) { return alloc_levels(c->d, c->mg, c->mg_n, true); }
+int cad_mg_alloc(cad_ctx *c) { return alloc_levels(c->d, c->mg, c->mg_n); }
 
 // the hierarchy of the context's current matrix.  Outside the K planes that
 // hold active cells every row is inactive (INDC = -1 there), as a freshly
@@ -870,10 +850,14 @@ int cad_mg_apply_resid(cad_ctx *c, const double *y, double *x, double *r, double
     return vcycle(c, c->mg, c->mg_n, y, x, k0, k1, r, part, stride);
 }
 
-int cad_mg_apply32(cad_ctx *c, const float *y, float *x, int k0, int k1)
+int cad_mg_cycle(cad_ctx *c, float *b, float *x)
 {
+    MgLevel mg[CAD_MG_MAX];
+    std::copy(c->mg, c->mg + c->mg_n, mg);
+    mg[0].b = b;
+    mg[0].x = x;
     RET_IF(cad_kt_begin(c, CAD_KT_VCYCLE));
-    RET_IF(vcycle(c, c->mg, c->mg_n, y, x, k0, k1));
+    RET_IF(passes(c, mg, c->mg_n, c->mg_k0, c->mg_k1));
     double by = 0.0;
     if (c->kt && c->kt->on) {
         Dims dims[CAD_MG_MAX];
@@ -884,7 +868,7 @@ int cad_mg_apply32(cad_ctx *c, const float *y, float *x, int k0, int k1)
 }
 
 // One V-cycle on the hierarchy and K range of the last mixed or learned
-// solve, timed with HIP events on the library's stream (input BB, output AE),
+// solve, timed with HIP events on the library's stream (right-hand side BB),
 // with its algorithmic bytes (vcycle_bytes); fp64 != 0: the same V-cycle with
 // every level in FP64 (a hierarchy of its own, built from the same matrix),
 // for comparison.
@@ -896,18 +880,24 @@ int cad_mg_time(cad_ctx *c, int reps, int fp64, float *ms_avg, double *bytes)
     }
     if (reps < 1) reps = 1;
     if (fp64) {
-        RET_IF(alloc_levels(c->d, c->mg64, c->mg64_n, false));
+        RET_IF(alloc_levels(c->d, c->mg64, c->mg64_n));
         RET_IF(setup_levels(c, c->mg64, c->mg64_n, 1, c->d.nk));
     }
+    const dim3 g = lvl_grid(c->d, c->mg_k0, c->mg_k1), tb(64, 4, 1);
+    if (fp64)
+        hipLaunchKernelGGL((k_mg_in<double, double>), g, tb, 0, c->stream, c->mg64[0], c->bb, c->mg_k0);
+    else
+        hipLaunchKernelGGL((k_mg_in<float, double>), g, tb, 0, c->stream, c->mg[0], c->bb, c->mg_k0);
+    CAD_CHECK(hipGetLastError());
     hipEvent_t a, b;
     CAD_CHECK(hipEventCreate(&a));
     CAD_CHECK(hipEventCreate(&b));
     CAD_CHECK(hipEventRecord(a, c->stream));
     for (int r = 0; r < reps; r++) {
         if (fp64)
-            RET_IF(vcycle(c, c->mg64, c->mg64_n, c->bb, c->ae, c->mg_k0, c->mg_k1));
+            RET_IF(passes(c, c->mg64, c->mg64_n, c->mg_k0, c->mg_k1));
         else
-            RET_IF(vcycle(c, c->mg, c->mg_n, c->bb, c->ae, c->mg_k0, c->mg_k1));
+            RET_IF(passes(c, c->mg, c->mg_n, c->mg_k0, c->mg_k1));
     }
     CAD_CHECK(hipEventRecord(b, c->stream));
     CAD_CHECK(hipEventSynchronize(b));

@@ -666,17 +666,17 @@ static int fetch_sc(cad_ctx *c, int slot, int n, double *out)
     return CAD_OK;
 }
 
-// Waits for the record {value, tag} that a kernel of the stream writes to the
-// context's pinned memory.
-static int wait_record(cad_ctx *c, int tag, double *out)
+// Waits for the record {value, tag} that a kernel of the stream writes to place
+// `at` of the context's pinned records.
+int cad_wait_record(cad_ctx *c, int at, double tag, double *out)
 {
-    const double *rec = c->host_red + CAD_REC;
+    const double *rec = c->host_red + CAD_REC + 2 * at;
     for (unsigned n = 1;; n++) {
         long long t;
         __atomic_load((const long long *)(rec + 1), &t, __ATOMIC_ACQUIRE);
         double v;
         std::memcpy(&v, &t, sizeof v);
-        if (v == (double)tag) break;
+        if (v == tag) break;
         if ((n & 0xFFFFu) == 0) {
             // an error, or a stream that has run dry without the record
             const hipError_t e = hipStreamQuery(c->stream);
@@ -684,7 +684,7 @@ static int wait_record(cad_ctx *c, int tag, double *out)
             CAD_CHECK(e);
             __atomic_load((const long long *)(rec + 1), &t, __ATOMIC_ACQUIRE);
             std::memcpy(&v, &t, sizeof v);
-            if (v == (double)tag) break;
+            if (v == tag) break;
             cad_set_error("the solve's stop record did not arrive");
             return CAD_ERR_HIP;
         }
@@ -835,7 +835,7 @@ int cad_solve_m1bcgs(cad_ctx *c, double *x0, double *bnorm_out, double *xnorm_ou
                 RET_IF_(rest());
             }
             if (spec)
-                RET_IF_(wait_record(c, iter, &xnorm));
+                RET_IF_(cad_wait_record(c, 0, (double)iter, &xnorm));
             else
                 RET_IF_(fetch_sc(c, SC_XN, 1, &xnorm));
             if (xnorm <= thr) {

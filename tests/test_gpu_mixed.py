@@ -138,3 +138,58 @@ def test_mixed_falls_back_to_milu_bicgstab(pkg):
     bn = info["cgbnrm"]
     assert res * bn <= (p["cgepsr"] * bn + p["cgepsa"]) * (1.0 + 1e-6)
     assert_close(f"{case} step {s} PT", pt, r["ps_out"]["PT"], 1e-6)
+
+
+# interior cells: whole solve in one workgroup with two rows of a colour a thread,
+# six, four; levels above it, odd extents; a coarsest level beyond it (two
+# lines and one line thick); over 2^20 cells; a half line just over 64 positions
+SHAPES = [(8, 8, 8), (25, 16, 12), (32, 16, 8), (97, 21, 13), (40, 33, 37), (300, 2, 40), (2, 130, 70),
+          (260, 70, 66), (129, 5, 4)]
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+def test_mixed_solve_over_level_shapes(pkg, shape):
+    """A Poisson system with a fixed value above a ragged surface, on grids whose
+    levels end in each kind of coarsest solve: three solves in a row (the
+    surface of the second is lower, the third is the first again) as captured
+    iterations and, with kernel timing on, as launches of their own give the
+    same bits; the true residual holds and no solve falls back.  Grids that
+    coarsen need few iterations, which a wrong row, correction or restriction
+    would not give."""
+    ni, nj, nk = (n + 2 for n in shape)
+    rs = np.random.default_rng(ni + nj)
+    systems = []
+    for level in (0.8, 0.5, 0.8):
+        indc = np.full((ni, nj, nk), -1, np.int32, order="F")
+        top = np.clip((level * shape[2] + rs.integers(-1, 2, shape[:2])).astype(int), 1, shape[2])
+        indc[1:-1, 1:-1, 1:-1] = np.where(np.arange(shape[2]) < top[:, :, None], 0, -1)
+        on = indc == 0
+        mat = {k: np.zeros((ni, nj, nk), order="F") for k in pkg.capi.MATRIX}
+        for a, (lo, up) in enumerate((("ALI", "AUI"), ("ALJ", "AUJ"), ("ALK", "AUK"))):
+            mat[lo][...] = np.where(on & np.roll(on, 1, axis=a), -1.0, 0.0)
+            mat[up][...] = np.where(on & np.roll(on, -1, axis=a), -1.0, 0.0)
+        above = on & ~np.roll(on, -1, axis=2)
+        mat["AD"][...] = np.where(on, above * 2.0 - sum(mat[k] for k in ("ALI", "AUI", "ALJ", "AUJ", "ALK", "AUK")), 0.0)
+        mat["BB"][...] = np.where(on, rs.standard_normal((ni, nj, nk)), 0.0)
+        systems.append((mat, indc))
+    lay = pkg.layout.from_text(pkg.configs.dam_break(*shape, col_x=0.01, col_z=0.01).deck)
+    outs = []
+    for timing in (0, 1):
+        with pkg.capi.Context(ni, nj, nk, lay.numb) as c:
+            c.upload_static(lay.static_arrays())
+            c.upload_state(lay.raw_state())
+            c.set_params(cgpara=0.95, icgtyp=1, cgepsa=0.0, cgepsr=1e-10, cgdiv=1e30, icgmax=2000,
+                         precision=pkg.capi.PRECISION_MIXED)
+            c.set_kernel_timing(timing)
+            for mat, indc in systems:
+                print(f"mixed {shape} timing {timing}", flush=True)
+                c.upload_matrix(mat, indc)
+                info = c.vpsol()
+                outs.append((info["icgitr"], c.poisson_residual(), c.download_pt()))
+            assert c.mixed_stats()["fallbacks"] == 0, shape
+    print(f"  ITR {[o[0] for o in outs]} residuals {[o[1] for o in outs]}", flush=True)
+    for a, b in zip(outs[:3], outs[3:]):
+        assert a[0] == b[0] and np.array_equal(a[2], b[2]), shape
+        assert a[1] <= 1e-10 * (1 + 1e-6), (shape, a[1])
+        if min(shape) >= 4:
+            assert a[0] <= 24, (shape, a[0])
