@@ -23,8 +23,8 @@
 // launches an iteration before it has read the last one's record where the
 // residuals' trend says that it will be needed (never a second one, so two records in
 // turn hold what it has not read); one launched beyond the stop changes nothing.
-// An iteration measured 240 us as 38 launches and a host
-// read on 97x61x45 cells, 125 as 22 in a graph; 880 and 700 on 512x256x128.
+// With all this 20 steps of drops on 97x61x45 cells take 52 ms instead of 70, ten of a tank
+// with buildings on 512x256x128 155 instead of 176.
 //
 // The inner solve stops at a relative residual eta = max(1e-6, 0.1
 // tol / ||r||): about what FP32 can resolve, and on the last outer step a

@@ -13,12 +13,12 @@
 //
 // Tiles.  A workgroup has one or two walking waves of 16 (J) x 4 (K) lines
 // along I, stacked in K, a helper wave for each, and two receivers.  Lane
-// jl + 16 kl walks line (J,K) with a skew of jl + 4 kl steps: its cell of step
-// (diagonal) d is I = d - jl - 4 kl.  The J neighbour is then lane jl-1's value of
+// jl + 16 kl walks line (J,K) with a skew of jl + 2 kl steps: its cell of step
+// (diagonal) d is I = d - jl - 2 kl.  The J neighbour is then lane jl-1's value of
 // the last step, one DPP row shift (lanes jl = 0 keep the halo value that the
-// shift leaves in place).  The K neighbour is lane kl-1's value of four steps
-// before: every pair of steps goes to a ring in LDS with one 16-byte write and
-// comes back with one read, issued a pair before it is needed; lanes kl = 0 read
+// shift leaves in place).  The K neighbour is lane kl-1's value of two steps
+// before: every step's value goes to a ring in LDS and comes back with a read
+// issued behind the write, a step before it is needed; lanes kl = 0 read
 // the halo ring at the same offsets.  A backward sweep walks the same diagonals
 // downwards with the roles of the first and last lanes swapped.
 //
@@ -44,11 +44,13 @@
 // flag that the host reports.
 //
 // What bounds it: a step is 65-80 ns, about 20 instructions and, with two walking
-// waves on a CU, the L1's 64 bytes a cycle; a tile-to-tile handover costs 3.5-5 us,
-// half of it the steps of the skew, half the way through memory.  M^-1 on water
+// waves on a CU, the L1's 64 bytes a cycle; a tile-to-tile handover costs 2.5-3.5 us,
+// a third of it the steps of the skew, the rest the way through memory.  With a skew of
+// four steps between K rows (values through the ring in pairs) M^-1 took 55 us on
+// 64x16x48 and 382 on 512x256x128, with two 46 and 368.  M^-1 on water
 // of the workloads, against the 64-line tiles of cad_sweep.hip (whose step was 240
-// ns, waiting for its mailbox accesses): buildings 512x256x128 660 -> 382 us, run-up
-// 512x32x96 330 -> 182, 250x70x90 267 -> 164, dam break 64x16x48 61 -> 55.  Those
+// ns, waiting for its mailbox accesses): buildings 512x256x128 660 -> 368 us, run-up
+// 512x32x96 330 -> 172, 250x70x90 267 -> 149, dam break 64x16x48 61 -> 46.  Those
 // tiles stay for the factorisation, for the fixed tile shapes, and where these
 // arrays do not fit.
 #include "cad_common.h"
@@ -62,7 +64,7 @@ namespace {
 typedef double v2d __attribute__((ext_vector_type(2)));
 
 constexpr int TJ = 16, TKW = 4;                  // lines of a wave in J and K
-constexpr int DK = 4;                            // steps between a wave's K rows
+constexpr int DK = 2;                            // steps between a wave's K rows
 constexpr int SKMAX = (TJ - 1) + DK * (TKW - 1);   // largest skew in a wave
 constexpr int S = 8, PQ = S / 2;                 // steps and step pairs of a stage
 constexpr int KOFF = DK * (TKW - 1);             // diagonals between a wave's first and last K row
@@ -523,8 +525,8 @@ __global__ void __launch_bounds__(64 * waves(NW), 1) k_wave(WGeom g, WCtl c, Op 
 #pragma unroll
         for (int q = 0; q < PQ; q++) fetch(fetch_lo(u), fetch_so(u), q, buf[u][q]);
 
-    // where this lane's K neighbour comes from: the own wave's ring two pairs
-    // back, the K halo ring, or the first wave's ring six pairs on
+    // where this lane's K neighbour comes from: the own wave's ring a pair back,
+    // the K halo ring, or the first wave's ring three pairs on
     char *const lds = reinterpret_cast<char *>(&sm);
     const char *kbase;
     int koff;
@@ -545,17 +547,16 @@ __global__ void __launch_bounds__(64 * waves(NW), 1) k_wave(WGeom g, WCtl c, Op 
     int *const mine = &sm.done[o][lane];
     v2d kq[PQ], jq[PQ], yq[PQ];
     auto kaddr = [&](int p) { return kb + ((p + koff) & (RX * PQ - 1)) * SLOT; };
-    // halo and Y of pair q of stage m; ka: the K address of the pair's half stage
-    auto halo = [&](int m, int q, int ka) {
-        kq[q] = *reinterpret_cast<const v2d *>(lds + ka + (q & 1) * SLOT);
+    // J halo and Y of pair q of stage m
+    auto halo = [&](int m, int q) {
         jq[q] = *reinterpret_cast<const v2d *>(&sm.jr[o][(m & (RX - 1)) * PQ + q][kl][0]);
         if (FWD) yq[q] = *reinterpret_cast<const v2d *>(yb + ((m & (RY - 1)) * PQ + q) * SLOT);
     };
     bool late = false;
     // whether stage m may be read and the ring has room for it (a: in[o], b: the
-    // other wave's stages).  Wave 1 reads wave 0's pairs up to six on from its
-    // stage's last; wave 0 must not overtake it by the ring.
-    const int ahead = NW == 1 ? INT_MIN / 2 : o == 0 ? 1 - RX : 3;
+    // other wave's stages).  Wave 1 reads wave 0's stage m + 1 during its own
+    // stage m; wave 0 must not overtake it by the ring.
+    const int ahead = NW == 1 ? INT_MIN / 2 : o == 0 ? 1 - RX : 2;
     auto allowed = [&](int4 a, int b, int m) {
         const int k = __builtin_amdgcn_readfirstlane(a.x), j = __builtin_amdgcn_readfirstlane(a.y);
         const int y = __builtin_amdgcn_readfirstlane(a.z), h = __builtin_amdgcn_readfirstlane(a.w);
@@ -574,11 +575,9 @@ __global__ void __launch_bounds__(64 * waves(NW), 1) k_wave(WGeom g, WCtl c, Op 
         order_lds();
     };
     wait_for(0);
-    {
-        const int ka = kaddr(0);
-        halo(0, 0, ka);
-        halo(0, 1, ka);
-    }
+    kq[0] = *reinterpret_cast<const v2d *>(lds + kaddr(0));
+    halo(0, 0);
+    halo(0, 1);
 
     // Two stages a turn; an odd walk ends with a stage of zeros.
     double x = 0.0;
@@ -588,13 +587,14 @@ __global__ void __launch_bounds__(64 * waves(NW), 1) k_wave(WGeom g, WCtl c, Op 
             const int m = m0 + u;
             const unsigned flo = fetch_lo(m + 2);
             const int fso = fetch_so(m + 2);
-            const int ka1 = kaddr(PQ * m + 2), ka2 = kaddr(PQ * m + 4);
+            // the K neighbours' pairs PQ m + 1 .. 3 lie in one stage's slots
+            const int ka1 = kaddr(PQ * m + 1), ka2 = kaddr(PQ * m + 4);
             char *const xs = xw + (m & (RX - 1)) * (PQ * SLOT);
             int4 fa;
             int fb;
 #pragma unroll
             for (int q = 0; q < PQ; q++) {
-                v2d xp;
+                const char *const kn = lds + (q < PQ - 1 ? ka1 + q * SLOT : ka2);
 #pragma unroll
                 for (int t = 0; t < 2; t++) {
                     const int h = FWD ? t : 1 - t;   // physical step of the pair
@@ -603,16 +603,18 @@ __global__ void __launch_bounds__(64 * waves(NW), 1) k_wave(WGeom g, WCtl c, Op 
                     for (int a = 0; a < NP; a++) v[a] = buf[u][q][a][h];
                     const double xj = from_j<DIR>(jq[q][t], x);
                     x = Op::step(v, FWD ? yq[q][t] : 0.0, x, xj, kq[q][t]);
-                    xp[t] = x;
+                    // and the same step's K value of the next pair
+                    *reinterpret_cast<double *>(xs + q * SLOT + 8 * t) = x;
+                    order_lds();
+                    kq[(q + 1) & (PQ - 1)][t] = *reinterpret_cast<const double *>(kn + 8 * t);
                 }
-                *reinterpret_cast<v2d *>(xs + q * SLOT) = xp;
                 fetch(flo, fso, q, buf[u][q]);
                 // the pair after next
                 order_lds();
                 if (q < 2)
-                    halo(m, q + 2, ka1);
+                    halo(m, q + 2);
                 else
-                    halo(m + 1, q - 2, ka2);
+                    halo(m + 1, q - 2);
                 if (q == 0) {
                     fa = *reinterpret_cast<const int4 *>(f);
                     fb = *other;
@@ -625,7 +627,7 @@ __global__ void __launch_bounds__(64 * waves(NW), 1) k_wave(WGeom g, WCtl c, Op 
         }
     }
     if (o == 0) {
-        // the second wave reads up to six pairs past the last stage: the lines
+        // the second wave reads up to three pairs past the last stage: the lines
         // hold no active cell there
         const int mz = (nst + 1) / 2 * 2;
         wait_for(mz + 1);
@@ -791,10 +793,10 @@ bool wave_geometry(const Dims &d, cad_wsweep *ws, WSizes *z)
     // One walking wave a workgroup has its CU's cache bandwidth to itself, two
     // share it but hand over in LDS what one would through memory.  Walks of
     // few steps are bound by the handovers, long or wide ones by the steps: on
-    // dam breaks (I x J x K) two against one measured 55 / 63 us on 64x16x48, 82 / 85 on
-    // 64x64x48, 104 / 102 on 128x48x64, 116 / 114 on 64x128x48, 114 / 106 on
-    // 512x16x64, 185 / 161 on 512x100x64.
-    const int nw = ws->nw = d.ni * d.nj >= 6000 ? 1 : 2;
+    // dam breaks (I x J x K) two against one measured 46 / 53 us on 64x16x48, 71 / 76 on
+    // 64x64x48, 91 / 92 on 128x48x64, 98 / 96 on 512x16x64, 136 / 136 on 512x32x96,
+    // 143 / 141 on 250x70x90, 165 / 149 on 512x100x64, 461 / 347 on 512x256x128.
+    const int nw = ws->nw = d.ni * d.nj >= 16000 ? 1 : 2;
     WGeom &g = ws->g;
     g.ni = d.ni;
     g.nj = d.nj;
