@@ -125,6 +125,9 @@ inline dim3 cell_grid(const Dims &d)
 // writes one partial, one block sums the partials in index order.
 constexpr int REDUCE_BLOCKS = 1024;
 constexpr int REDUCE_THREADS = 256;
+// a block's place among n (a multiple of 8) when the blocks that the eight XCDs
+// take in turn are put next to each other
+__device__ __forceinline__ int xcd_block(int n) { return (int)(blockIdx.x & 7u) * (n >> 3) + (int)(blockIdx.x >> 3); }
 constexpr int REDUCE_SLOTS = 6;   // products whose partials are kept apart
 constexpr int CAD_REC = 8;        // first double of the solves' records in host_red
 

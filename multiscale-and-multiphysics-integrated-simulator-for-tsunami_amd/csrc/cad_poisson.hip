@@ -245,6 +245,14 @@ __global__ void k_range_init(unsigned long long *rng, long long nc, double *sc)
     for (long long n = n0_ + (long long)blockIdx.x * blockDim.x + threadIdx.x; n < n1_; \
          n += (long long)(nblocks) * blockDim.x)
 
+// The same with the blocks of an XCD (blockIdx.x % 8) next to each other, for
+// kernels that read neighbouring lines: the lines of the blocks around it are then in
+// its L2.
+#define STENCIL_LOOP(n, rng, nblocks)                                                  \
+    const long long n0_ = (long long)(rng)[0], n1_ = (long long)(rng)[1];           \
+    for (long long n = n0_ + (long long)xcd_block(nblocks) * blockDim.x + threadIdx.x; n < n1_; \
+         n += (long long)(nblocks) * blockDim.x)
+
 // y = A x on active cells, vf_mzax.f:42-56 (active cells are interior, so all
 // seven neighbours exist)
 __global__ void __launch_bounds__(256) k_mzax(Dims d, const unsigned long long *rng,
@@ -259,7 +267,7 @@ __global__ void __launch_bounds__(256) k_mzax(Dims d, const unsigned long long *
                                               const double *__restrict__ x, double *__restrict__ y)
 {
     const long long ni = d.ni, nij = d.nij;
-    ACTIVE_LOOP(n, rng, VEC_BLOCKS) {
+    STENCIL_LOOP(n, rng, VEC_BLOCKS) {
         if (indc[n] == -1) continue;
         y[n] = ad[n] * x[n] + ali[n] * x[n - 1] + alj[n] * x[n - ni] + alk[n] * x[n - nij]
              + aui[n] * x[n + 1] + auj[n] * x[n + ni] + auk[n] * x[n + nij];
@@ -349,9 +357,9 @@ __device__ __forceinline__ void final_sums(const double *__restrict__ partial, d
 }
 
 // a block whose share of the active range is empty
-__device__ __forceinline__ bool idle_block(const unsigned long long *rng)
+__device__ __forceinline__ bool idle_block(const unsigned long long *rng, int block)
 {
-    return rng[0] + (unsigned long long)blockIdx.x * blockDim.x >= rng[1];
+    return rng[0] + (unsigned long long)block * blockDim.x >= rng[1];
 }
 
 // x += alpha p + omega r ; r -= omega ae ; partials of (r, r) and (r0, r),
@@ -367,7 +375,7 @@ __global__ void __launch_bounds__(REDUCE_THREADS) k_update_xr(const unsigned lon
                                                               double *partial)
 {
     if (sc[SC_DONE] != 0.0) return;
-    if (blockIdx.x != 0 && idle_block(rng)) {
+    if (blockIdx.x != 0 && idle_block(rng, (int)blockIdx.x)) {
         if (threadIdx.x < 2) partial[threadIdx.x * REDUCE_BLOCKS + blockIdx.x] = 0.0;
         return;
     }
@@ -406,14 +414,14 @@ __global__ void __launch_bounds__(REDUCE_THREADS) k_s_ax(Dims d, const unsigned 
                                                          const double *__restrict__ ap,
                                                          double *__restrict__ s, double *__restrict__ y)
 {
-    if (sc[SC_DONE] != 0.0 || (blockIdx.x != 0 && idle_block(rng))) return;
+    if (sc[SC_DONE] != 0.0 || (blockIdx.x != 0 && idle_block(rng, xcd_block(VEC_BLOCKS)))) return;
     double w[1];
     final_sums<1>(w1_part, w);
     const double alpha = sc[s_slot] / w[0];
     if (blockIdx.x == 0 && threadIdx.x == 0) sc[SC_ALPHA] = alpha;
     const long long ni = d.ni, nij = d.nij;
     auto v = [&](long long n) { return r[n] - alpha * ap[n]; };
-    ACTIVE_LOOP(n, rng, VEC_BLOCKS) {
+    STENCIL_LOOP(n, rng, VEC_BLOCKS) {
         if (indc[n] == -1) continue;
         const double c = v(n);
         s[n] = c;
@@ -442,7 +450,7 @@ __global__ void __launch_bounds__(REDUCE_THREADS) k_p_ax(Dims d, const unsigned 
                                                          const double *__restrict__ ap,
                                                          double *__restrict__ pn, double *__restrict__ y)
 {
-    if (blockIdx.x != 0 && idle_block(rng)) return;
+    if (blockIdx.x != 0 && idle_block(rng, xcd_block(VEC_BLOCKS))) return;
     double w[2];
     final_sums<2>(xr_part, w);
     const bool stop = thr >= 0.0 && (w[0] <= thr || w[0] > div2);
@@ -460,7 +468,7 @@ __global__ void __launch_bounds__(REDUCE_THREADS) k_p_ax(Dims d, const unsigned 
     if (stop) return;
     const long long ni = d.ni, nij = d.nij;
     auto v = [&](long long n) { return r[n] + beta * (p[n] - omega * ap[n]); };
-    ACTIVE_LOOP(n, rng, VEC_BLOCKS) {
+    STENCIL_LOOP(n, rng, VEC_BLOCKS) {
         if (indc[n] == -1) continue;
         const double c = v(n);
         pn[n] = c;

@@ -237,7 +237,8 @@ __global__ void __launch_bounds__(REDUCE_THREADS) k_r_mv(MgLevel L, Tiles T, con
     if (sc[S_DONE] != 0.0) return;
     const int lj = L.ld, lk = L.ld * L.d.nj, half = L.ld >> 1;
     double a[2] = {0.0, 0.0};
-    for (int t = blockIdx.x; t < T.n; t += gridDim.x) {
+    const int b0 = gridDim.x % 8 == 0 ? xcd_block(gridDim.x) : (int)blockIdx.x;
+    for (int t = b0; t < T.n; t += gridDim.x) {
         const int qt = t % T.qt, r1 = t / T.qt, color = r1 & 1, r2 = r1 >> 1, jt = r2 % T.jt, k = T.k0 + r2 / T.jt;
         const int q = qt * 64 + (int)(threadIdx.x & 63), j = jt * 4 + (int)(threadIdx.x >> 6) + 2;
         const int i = 2 * q + 1 + ((color + 1 + j + k) & 1);
