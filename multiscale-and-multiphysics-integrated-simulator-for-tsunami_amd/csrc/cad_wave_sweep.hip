@@ -33,8 +33,9 @@
 // mailbox entries, written by the helpers, never waited for.  They are indexed
 // by the consumer's own diagonal, so a stage of a tile's K halo is 2 KB
 // contiguous and of a wave's J halo 512 bytes.  The receivers (one for the K
-// halo, one for the J halos) poll them, several stages at a time once
-// values flow, and put them into rings; a second walking wave reads the first
+// halo, one for the J halos) poll them a stage at a time and put them into rings
+// (a poll's latency grows with its cache lines: polls of two stages ahead
+// made M^-1 9 % slower on 512x256x128, three polls in flight 14 to 25 %); a second walking wave reads the first
 // one's ring.  All waves keep pace by stage counters in LDS, which a walking wave
 // looks at once a stage, a stage ahead.  LDS operations of a wave execute in
 // order, so a counter written after its values is seen after them.
@@ -44,13 +45,14 @@
 // flag that the host reports.
 //
 // What bounds it: a step is 65-80 ns, about 20 instructions and, with two walking
-// waves on a CU, the L1's 64 bytes a cycle; a tile-to-tile handover costs 2.5-3.5 us,
-// a third of it the steps of the skew, the rest the way through memory.  With a skew of
+// waves on a CU, the L1's 64 bytes a cycle; a tile-to-tile handover costs 2-3 us,
+// half of it the steps of the skew, the rest the way through memory.  With a skew of
 // four steps between K rows (values through the ring in pairs) M^-1 took 55 us on
-// 64x16x48 and 382 on 512x256x128, with two 46 and 368.  M^-1 on water
+// 64x16x48 and 382 on 512x256x128, with two 46 and 368, with polls of one stage
+// and the J halo whole in its own entries 43 and 312.  M^-1 on water
 // of the workloads, against the 64-line tiles of cad_sweep.hip (whose step was 240
-// ns, waiting for its mailbox accesses): buildings 512x256x128 660 -> 368 us, run-up
-// 512x32x96 330 -> 172, 250x70x90 267 -> 149, dam break 64x16x48 61 -> 46.  Those
+// ns, waiting for its mailbox accesses): buildings 512x256x128 661 -> 312 us, run-up
+// 512x32x96 330 -> 155, 250x70x90 267 -> 129, dam break 64x16x48 61 -> 43.  Those
 // tiles stay for the factorisation, for the fixed tile shapes, and where these
 // arrays do not fit.
 #include "cad_common.h"
@@ -186,58 +188,45 @@ __device__ void receive_k(WSmem<NW> &sm, const WGeom &g, const WCtl &c, int bj, 
     const int lo = pr.x / S * S, hi = (pr.y + SKMAX) / S * S + S - 1;   // diagonals the producer walks
     const __amdgpu_buffer_rsrc_t r = rsrc(c.mb, c.mb_bytes);
     const unsigned base = (unsigned)(((pt * (g.nd + 2 * KPAD) + KPAD) * TJ + jl) * 16);
-    constexpr int CH = 4;
-    int m = 0;
-    bool flow = false, late = false;
+    bool late = false;
     unsigned spins = 0;
-    while (m < nst) {
-        const int nq = min(flow ? CH : 1, nst - m);
-        v3u e[CH][2];
-        bool need[CH][2];
+    for (int m = 0; m < nst;) {
+        v3u e[2];
+        bool need[2], ok = true;
 #pragma unroll
-        for (int q = 0; q < CH; q++)
-#pragma unroll
-            for (int h = 0; h < 2; h++) {
-                const int d1 = S * (s0 + DIR * (m + q)) + phys<DIR>(e0 + 4 * h), d = d1 + KOFF * DIR;
-                need[q][h] = q < nq && d >= lo && d <= hi;
-                e[q][h] = mb_load(r, need[q][h] ? base + (unsigned)(d1 * (TJ * 16)) : OOB);
-            }
-        int got = 0;
-#pragma unroll
-        for (int q = 0; q < CH; q++) {
-            if (q >= nq || got < q) continue;
-            const bool ok = (!need[q][0] || e[q][0].z == c.seq) && (!need[q][1] || e[q][1].z == c.seq);
-            if (__builtin_amdgcn_ballot_w64(!ok) != 0) continue;
-            unsigned n = 0;
-            while (!late && cnt_load(done) <= m + q - RX) {
-                __builtin_amdgcn_s_sleep(1);
-                if (++n > LDS_SPINS) late = true;
-            }
-            order_lds();
-            const int sl = ((m + q) & (RX - 1)) * PQ;
-#pragma unroll
-            for (int h = 0; h < 2; h++) {
-                const int w = e0 + 4 * h;
-                *reinterpret_cast<double *>(sm.kr + (sl + (w >> 1)) * SLOT + jl * 16 + (w & 1) * 8) =
-                    need[q][h] ? __builtin_bit_cast(double, v2u{e[q][h].x, e[q][h].y}) : 0.0;
-            }
-            got = q + 1;
+        for (int h = 0; h < 2; h++) {
+            const int d1 = S * (s0 + DIR * m) + phys<DIR>(e0 + 4 * h), d = d1 + KOFF * DIR;
+            need[h] = d >= lo && d <= hi;
+            e[h] = mb_load(r, need[h] ? base + (unsigned)(d1 * (TJ * 16)) : OOB);
         }
-        if (got) {
-            m += got;
-            order_lds();
-            if (lane == 0) cnt_store(flag, m);
-            order_lds();
-            flow = true;
-            spins = 0;
-        } else {
-            flow = false;
+#pragma unroll
+        for (int h = 0; h < 2; h++) ok = ok && (!need[h] || e[h].z == c.seq);
+        if (__builtin_amdgcn_ballot_w64(!ok) != 0) {
             __builtin_amdgcn_s_sleep(1);
             if ((++spins & 1023u) == 0u) {
                 if (spins > SPIN_LIMIT) atomicOr(c.err, 2);
                 if (__hip_atomic_load(c.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) break;
             }
+            continue;
         }
+        unsigned n = 0;
+        while (!late && cnt_load(done) <= m - RX) {
+            __builtin_amdgcn_s_sleep(1);
+            if (++n > LDS_SPINS) late = true;
+        }
+        order_lds();
+        const int sl = (m & (RX - 1)) * PQ;
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const int w = e0 + 4 * h;
+            *reinterpret_cast<double *>(sm.kr + (sl + (w >> 1)) * SLOT + jl * 16 + (w & 1) * 8) =
+                need[h] ? __builtin_bit_cast(double, v2u{e[h].x, e[h].y}) : 0.0;
+        }
+        m++;
+        spins = 0;
+        order_lds();
+        if (lane == 0) cnt_store(flag, m);
+        order_lds();
     }
     order_lds();
     if (lane == 0) cnt_store(flag, INT_MAX);
@@ -262,47 +251,27 @@ __device__ void receive_j(WSmem<NW> &sm, const WGeom &g, const WCtl &c, int bj, 
     }
     const int lo = pr.x / S * S, hi = (pr.y + SKMAX) / S * S + S - 1;
     const __amdgpu_buffer_rsrc_t r = rsrc(c.mb, c.mb_bytes);
-    // the second wave's last K row is published on the K side only, at the K
-    // consumer's diagonal
-    const bool corner = o == NW - 1 && kl == (DIR > 0 ? TKW - 1 : 0);
-    const unsigned base =
-        corner ? (unsigned)(((pt * (g.nd + 2 * KPAD) + KPAD + DIR * (TJ - 1 - KOFF)) * TJ + (DIR > 0 ? TJ - 1 : 0)) * 16)
-               : c.j_base + (unsigned)((((pt * NW + w) * (g.nd + 2 * JPAD) + JPAD) * TKW + kl) * 16);
-    const int pitch = corner ? TJ * 16 : TKW * 16;
-    constexpr int CH = 4;
+    const unsigned base = c.j_base + (unsigned)((((pt * NW + w) * (g.nd + 2 * JPAD) + JPAD) * TKW + kl) * 16);
     int m = 0;                       // stages ready, per half
-    bool flow = false;
     unsigned spins = 0;
     const unsigned long long half = o ? 0xFFFFFFFF00000000ull : 0x00000000FFFFFFFFull;
     while (__builtin_amdgcn_ballot_w64(m < nst) != 0) {
-        const int nq = min(flow ? CH : 1, nst - m);
-        v3u e[CH];
-        bool need[CH];
-#pragma unroll
-        for (int q = 0; q < CH; q++) {
-            const int d1 = S * (s0 + DIR * (m + q)) + phys<DIR>(e0), d = d1 + (TJ - 1) * DIR;
-            need[q] = q < nq && d >= lo && d <= hi;
-            e[q] = mb_load(r, need[q] ? base + (unsigned)(d1 * pitch) : OOB);
-        }
-        int got = 0;
+        const int d1 = S * (s0 + DIR * m) + phys<DIR>(e0), d = d1 + (TJ - 1) * DIR;
+        const bool need = m < nst && d >= lo && d <= hi;
+        const v3u e = mb_load(r, need ? base + (unsigned)(d1 * (TKW * 16)) : OOB);
         const int dn = cnt_load(done);
+        const bool ok = m < nst && (!need || e.z == c.seq) && dn > m - RX;
+        const bool got = (__builtin_amdgcn_ballot_w64(!ok) & half) == 0;
         order_lds();
-#pragma unroll
-        for (int q = 0; q < CH; q++) {
-            const bool ok = q < nq && (!need[q] || e[q].z == c.seq) && dn > m + q - RX;
-            const bool all = (__builtin_amdgcn_ballot_w64(!ok) & half) == 0;
-            if (all && got == q) {
-                const int sl = ((m + q) & (RX - 1)) * PQ + (e0 >> 1);
-                sm.jr[o][sl][kl][e0 & 1] = need[q] ? __builtin_bit_cast(double, v2u{e[q].x, e[q].y}) : 0.0;
-                got = q + 1;
-            }
+        if (got) {
+            sm.jr[o][(m & (RX - 1)) * PQ + (e0 >> 1)][kl][e0 & 1] =
+                need ? __builtin_bit_cast(double, v2u{e.x, e.y}) : 0.0;
+            m++;
         }
         order_lds();
-        m += got;
         if (got && (lane & 31) == 0) cnt_store(flag, m);
         order_lds();
-        flow = got > 0;
-        if (__builtin_amdgcn_ballot_w64(got > 0) == 0) {
+        if (__builtin_amdgcn_ballot_w64(got) == 0) {
             __builtin_amdgcn_s_sleep(1);
             if ((++spins & 1023u) == 0u) {
                 if (spins > SPIN_LIMIT) atomicOr(c.err, 2);
@@ -326,14 +295,12 @@ __device__ void help(WSmem<NW> &sm, const WGeom &g, const WCtl &c, const Op &op,
     constexpr bool FWD = DIR > 0;
     constexpr int JP = FWD ? TJ - 1 : 0, KP = FWD ? TKW - 1 : 0;   // publishing lanes
     const bool has_j = bj + DIR >= 0 && bj + DIR < g.ntj, has_k = bk + DIR >= 0 && bk + DIR < g.ntk;
-    // the second wave's last K row goes to the K side (and serves the corner of
-    // the J side)
-    const bool pub_k = o == NW - 1 && (has_k || has_j);
+    const bool pub_k = o == NW - 1 && has_k;
     const __amdgpu_buffer_rsrc_t rmb = rsrc(c.mb, c.mb_bytes);
     // K entries: lane = jl + 16 e0, walking steps e0 and e0 + 4; J: kl + 4 e
     const int e0 = lane >> 4, kj = lane & 3, ej = lane >> 2;
     const unsigned kbase = (unsigned)(((tile * (g.nd + 2 * KPAD) + KPAD - KOFF * DIR) * TJ + (lane & 15)) * 16);
-    const bool jlane = has_j && ej < S && !(o == NW - 1 && kj == KP);
+    const bool jlane = has_j && ej < S;
     const unsigned jbase =
         c.j_base + (unsigned)((((tile * NW + w) * (g.nd + 2 * JPAD) + JPAD - (TJ - 1) * DIR) * TKW + kj) * 16);
     // grid order: lane = pair + 4 (line % 16), lines in four groups of 16; in a
@@ -791,12 +758,12 @@ struct WSizes {
 bool wave_geometry(const Dims &d, cad_wsweep *ws, WSizes *z)
 {
     // One walking wave a workgroup has its CU's cache bandwidth to itself, two
-    // share it but hand over in LDS what one would through memory.  Walks of
-    // few steps are bound by the handovers, long or wide ones by the steps: on
-    // dam breaks (I x J x K) two against one measured 46 / 53 us on 64x16x48, 71 / 76 on
-    // 64x64x48, 91 / 92 on 128x48x64, 98 / 96 on 512x16x64, 136 / 136 on 512x32x96,
-    // 143 / 141 on 250x70x90, 165 / 149 on 512x100x64, 461 / 347 on 512x256x128.
-    const int nw = ws->nw = d.ni * d.nj >= 16000 ? 1 : 2;
+    // share it but hand over in LDS what one would through memory, which pays
+    // where walks are short and the K rows many: on
+    // dam breaks (I x J x K) two against one measured 25 / 22 us on 30x16x16, 43 / 48 on
+    // 64x16x48, 68 / 68 on 64x64x48, 87 / 83 on 128x48x64, 91 / 88 on 512x16x64,
+    // 133 / 127 on 250x70x90, 149 / 133 on 512x100x64, 414 / 305 on 512x256x128.
+    const int nw = ws->nw = d.ni * d.nj < 4096 && d.nk >= 32 ? 2 : 1;
     WGeom &g = ws->g;
     g.ni = d.ni;
     g.nj = d.nj;
