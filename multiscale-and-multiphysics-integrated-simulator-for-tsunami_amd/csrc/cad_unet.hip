@@ -72,12 +72,6 @@ __device__ __forceinline__ long long vox_of(const UGeo &g, long long u)
     return vox(g, x, y, z, b);
 }
 
-__device__ __forceinline__ long long tap_off(const UGeo &g, int t)
-{
-    const int dx = t % 3 - 1, dy = (t / 3) % 3 - 1, dz = t / 9 - 1;
-    return dx + (long long)g.px * (dy + (long long)g.py * dz);
-}
-
 // K steps of 32 of the folded convolution for cin input channels (9 taps)
 __host__ __device__ constexpr int fold_kc(int cin) { return (9 * cin + 31) / 32; }
 // bytes of A fragments a launch of MT channel tiles stages in LDS, and the cap
