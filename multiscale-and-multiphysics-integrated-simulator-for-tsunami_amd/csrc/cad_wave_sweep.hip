@@ -232,11 +232,15 @@ __device__ void receive_k(WSmem<NW> &sm, const WGeom &g, const WCtl &c, int bj, 
     if (lane == 0) cnt_store(flag, INT_MAX);
 }
 
-// The J receiver: lanes 0..31 serve walking wave 0, lanes 32..63 wave 1.
+// The J receiver: lanes 0..31 serve walking wave 0, lanes 32..63 wave 1.  With one
+// walking wave the upper lanes leave: a lane's load is its own, served at a time of
+// its own, so a second lane with the same entry would store a value whose
+// sequence number nobody has looked at.
 template <int DIR, int NW>
 __device__ void receive_j(WSmem<NW> &sm, const WGeom &g, const WCtl &c, int bj, int bk, int s0, int nst, int lane)
 {
-    const int o = min(lane >> 5, NW - 1), w = DIR > 0 ? o : NW - 1 - o;
+    if (lane >= 32 * NW) return;
+    const int o = lane >> 5, w = DIR > 0 ? o : NW - 1 - o;
     int *flag = &sm.in[o][1];
     const int *done = &sm.done[o][0];
     const int pbj = bj - DIR;
