@@ -229,7 +229,10 @@ __device__ void receive_k(WSmem<NW> &sm, const WGeom &g, const WCtl &c, int bj, 
         order_lds();
     }
     order_lds();
-    if (lane == 0) cnt_store(flag, INT_MAX);
+    if (lane == 0) {
+        cnt_store(flag, INT_MAX);
+        if (late) atomicOr(c.err, 2);
+    }
 }
 
 // The J receiver: lanes 0..31 serve walking wave 0, lanes 32..63 wave 1.  With one

@@ -31,3 +31,12 @@ def test_receivers_take_only_checked_values(receivers, which, way, nw):
     for seed in range(12):
         r = subprocess.run([receivers, which, way, str(nw), str(seed)], capture_output=True, text=True, timeout=60)
         assert r.returncode == 0, (seed, r.stdout)
+
+
+@pytest.mark.parametrize("nw", [1, 2])
+@pytest.mark.parametrize("way", ["fwd", "bwd"])
+def test_ring_space_that_never_comes_sets_the_error_flag(receivers, way, nw):
+    """A walking wave that stands still: the K receiver's wait for room in the ring
+    ends, and the launch's error flag says so."""
+    r = subprocess.run([receivers, "stuck", way, str(nw)], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, r.stdout
