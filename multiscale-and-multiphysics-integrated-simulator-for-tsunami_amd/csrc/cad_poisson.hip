@@ -847,10 +847,17 @@ int cad_solve_m1bcgs(cad_ctx *c, double *x0, double *bnorm_out, double *xnorm_ou
                 RET_IF_(cad_wait_record(c, 0, (double)iter, &xnorm));
             else
                 RET_IF_(fetch_sc(c, SC_XN, 1, &xnorm));
-            if (xnorm <= thr) {
+            const bool below = xnorm <= thr;
+            if (below) {
                 bool ok = true;
                 if (true_stop) RET_IF_(true_ok(&ok));
                 if (ok) break;
+            }
+            if (xnorm > div2) {
+                iter = -2;
+                break;
+            }
+            if (below) {
                 // the true residual does not hold yet: this iteration again,
                 // without the test
                 p = p0;
@@ -863,9 +870,6 @@ int cad_solve_m1bcgs(cad_ctx *c, double *x0, double *bnorm_out, double *xnorm_ou
                     advance();
                     RET_IF_(rest());
                 }
-            } else if (xnorm > div2) {
-                iter = -2;
-                break;
             } else if (!ahead) {
                 advance();
                 if (iter < c->prm.icgmax) RET_IF_(rest());

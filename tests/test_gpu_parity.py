@@ -221,3 +221,22 @@ def test_true_residual_stop(pkg, case):
         assert info["icgitr"] >= int(r["ps_out"]["ICGITR"][0])
         assert res <= 1e-11, res
         assert_close(f"{case} step {s} PT", pt, r["ps_out"]["PT"], 1e-8)
+
+
+@pytest.mark.parametrize("timing", [0, 1])
+def test_divergence_is_tested_where_only_the_true_residual_holds_a_solve(pkg, timing):
+    """An iterate that passes the preconditioned test but not the true residual's
+    goes on to the divergence test (the loop of vf_m1bcgs.f:101-262), also with the host an
+    iteration behind (timing 0)."""
+    case = "tiny"
+    st = fx.static(case)
+    r = fx.step(case, fx.steps(case)[0])
+    with _ctx(pkg, case, st, r["v1_in"]) as c:
+        c.upload_state(_state(r["v1_in"], r["f1_in"]["BCF"]))
+        c.upload_matrix(r["ps_in"], r["ps_in"]["INDC"])
+        c.set_kernel_timing(timing)
+        c.set_true_residual_stop(1e-11)
+        c.set_params(cgepsr=2.0, cgdiv=1e-30)
+        with pytest.raises(pkg.capi.CadError) as e:
+            c.vpsol()
+    assert e.value.code == -31
