@@ -263,6 +263,7 @@ struct cad_ctx {
     int mg64_n;
     unsigned long long mg_span;   // cells in the active index range of the current solve
     int mg_k0, mg_k1;             // K planes of level 0's passes in the current solve
+    int mg_planes;                // those from the first to the last active cell, its counted work
     struct cad_mixed *mx;         // the mixed form's vectors and captured iteration (cad_refine.hip)
     int mg_set_k0, mg_set_k1;     // K planes level 0's rows were last built on (0: none yet)
     // the learned form's network, Krylov basis and counters (cad_learned.hip),

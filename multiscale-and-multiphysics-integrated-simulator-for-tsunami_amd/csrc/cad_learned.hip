@@ -610,6 +610,7 @@ int setup(cad_ctx *c, bool *empty)
     const int k1 = (int)((hr[1] - 1) / (unsigned long long)d.nij) + 1;
     c->mg_k0 = k0;
     c->mg_k1 = k1;
+    c->mg_planes = k1 - k0 + 1;
     if (L->mode == 1) RET_IF(cad_mg_setup(c));
     L->kb = k0;
     L->nzr = std::min(((k1 - k0 + 1) + 3) / 4 * 4, L->nzmax);

@@ -798,7 +798,9 @@ int vcycle(cad_ctx *c, const MgLevelT<V> *mg, int nl, const T *y, T *x, int k0, 
 // neighbours read once: 10 values + 1 byte per cell and colour pair), the
 // residual-restriction of the even cells (7 coefficients, b, x, activity,
 // and a share of the coarse b and x) and the coarse x that the corrected
-// even half-sweep reads; on the coarsest level MG_COARSE full sweeps.
+// even half-sweep reads; on the coarsest level MG_COARSE full sweeps.  Level 0
+// counts with the planes from the first to the last active cell, also where its
+// passes run on more.
 double vcycle_bytes(const cad_ctx *c, const Dims *dims, int nl, int vs)
 {
     const double half = (10.0 * vs + 1.0) / 2.0;
@@ -807,7 +809,7 @@ double vcycle_bytes(const cad_ctx *c, const Dims *dims, int nl, int vs)
     double by = 0.0;
     for (int l = 0; l < nl; l++) {
         const Dims &d = dims[l];
-        const int planes = l == 0 ? c->mg_k1 - c->mg_k0 + 1 : d.nk - 2;
+        const int planes = l == 0 ? c->mg_planes : d.nk - 2;
         const double cells = (double)(d.ni - 2) * (double)(d.nj - 2) * (double)planes;
         by += l == nl - 1 ? 2.0 * half * MG_COARSE * cells : (3.0 * half + restr + prol) * cells;
     }

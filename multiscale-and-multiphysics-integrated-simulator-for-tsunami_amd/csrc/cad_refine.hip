@@ -523,9 +523,11 @@ int cad_solve_mixed(cad_ctx *c, double *x0, double *bnorm_out, double *xnorm_out
     // level 0's planes: those with active cells, widened to fours so that a
     // moving surface seldom asks for another graph (the planes between hold
     // inactive rows only)
+    const int ka = (int)(hr[0] / (unsigned long long)d.nij) + 1, kb = (int)((hr[1] - 1) / (unsigned long long)d.nij) + 1;
     c->mg_span = hr[1] - hr[0];
-    c->mg_k0 = std::max(2, (int)(hr[0] / (unsigned long long)d.nij + 1) & ~3);
-    c->mg_k1 = std::min(d.nk - 1, (int)((hr[1] - 1) / (unsigned long long)d.nij + 1) | 3);
+    c->mg_planes = kb - ka + 1;
+    c->mg_k0 = std::max(2, ka & ~3);
+    c->mg_k1 = std::min(d.nk - 1, kb | 3);
     RET_IF(cad_mg_setup(c));
     RET_IF(mixed_alloc(c));
     const MgLevel &L0 = c->mg[0];

@@ -89,3 +89,42 @@ def test_kernel_timing_counts_launches_and_changes_nothing(pkg, form):
         assert n >= 1 and ms > 0.0
         assert work == on["iso"][1]
         assert counts["vcycle"] == 0
+
+
+def test_vcycle_bytes_count_the_planes_with_active_cells(pkg):
+    """The V-cycle's algorithmic bytes, from cad_time_precond and per launch from the
+    in-solve timing, count level 0 on the planes that hold active cells: here the
+    third to the fifth of twenty, though its passes run on planes in fours."""
+    shape = (40, 12, 20)
+    ni, nj, nk = (n + 2 for n in shape)
+    indc = np.full((ni, nj, nk), -1, np.int32, order="F")
+    indc[1:-1, 1:-1, 3:6] = 0
+    on = indc == 0
+    mat = {k: np.zeros((ni, nj, nk), order="F") for k in pkg.capi.MATRIX}
+    for a, (lo, up) in enumerate((("ALI", "AUI"), ("ALJ", "AUJ"), ("ALK", "AUK"))):
+        mat[lo][...] = np.where(on & np.roll(on, 1, axis=a), -1.0, 0.0)
+        mat[up][...] = np.where(on & np.roll(on, -1, axis=a), -1.0, 0.0)
+    mat["AD"][...] = np.where(on, 6.5, 0.0)
+    mat["BB"][...] = np.where(on, np.random.default_rng(3).standard_normal((ni, nj, nk)), 0.0)
+    # per cell of a level above the coarsest: three half-sweeps, the restriction
+    # of the even cells, the coarse x of the corrected half-sweep; there 12 sweeps
+    half, restr, prol = 41.0 / 2.0, 37.0 / 2.0 + 1.0, 0.5
+    dims = [shape]
+    while min(dims[-1]) >= 4:
+        dims.append(tuple((n + 1) // 2 for n in dims[-1]))
+    dims[0] = (40, 12, 3)
+    want = sum(np.prod(d) * (24.0 * half if d is dims[-1] else 3.0 * half + restr + prol) for d in dims)
+    lay = pkg.layout.from_text(pkg.configs.dam_break(*shape, col_x=0.01, col_z=0.01).deck)
+    with pkg.capi.Context(ni, nj, nk, lay.numb) as c:
+        c.upload_static(lay.static_arrays())
+        c.upload_state(lay.raw_state())
+        c.set_params(cgpara=0.95, icgtyp=1, cgepsa=0.0, cgepsr=1e-8, cgdiv=1e30, icgmax=500,
+                     precision=pkg.capi.PRECISION_MIXED)
+        c.set_kernel_timing(1)
+        c.upload_matrix(mat, indc)
+        c.vpsol()
+        c.set_kernel_timing(0)
+        _, work, n = c.kernel_timing(pkg.capi.KERNEL_VCYCLE)
+        _, iso = c.time_precond(1)
+    assert n > 0 and work == want, (work, want, n)
+    assert iso == want, (iso, want)
