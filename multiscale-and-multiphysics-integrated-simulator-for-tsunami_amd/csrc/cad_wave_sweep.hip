@@ -53,11 +53,12 @@
 // of the workloads, against the 64-line tiles of cad_sweep.hip (whose step was 240
 // ns, waiting for its mailbox accesses): buildings 512x256x128 661 -> 312 us, run-up
 // 512x32x96 330 -> 155, 250x70x90 267 -> 129, dam break 64x16x48 61 -> 43.  Those
-// tiles stay for the factorisation, for the fixed tile shapes, and where these
-// arrays do not fit.
+// tiles stay for the factorisation, for the fixed tile shapes, on tall columns, and
+// where these arrays do not fit.
 #include "cad_common.h"
 #include "cad_sweep.h"
 
+#include <algorithm>
 #include <climits>
 #include <new>
 
@@ -761,9 +762,16 @@ struct WSizes {
 };
 
 // the geometry and the arrays' sizes for a grid; false where 32-bit offsets do
-// not reach
+// not reach, and on tall columns
 bool wave_geometry(const Dims &d, cad_wsweep *ws, WSizes *z)
 {
+    // A tall column's sweep is a chain of tiles in K with next to no walk, and the
+    // 64-line tiles of cad_sweep.hip hand over in less time: M^-1 of those / of
+    // this file's in us, I x J x K: 105 / 147 on 2x2x200, 204 / 226 on 4x4x300,
+    // 235 / 247 on 40x8x300, 294 / 315 on 24x8x400, 554 / 600 on 6x30x800; equal on
+    // 24x8x200 and 12x40x400; 126 / 129 on 8x8x160, 135 / 120 on 20x20x128, 106 / 102 on
+    // 24x8x120.
+    if (d.nk - 2 >= 5 * std::max(d.ni - 2, d.nj - 2) + 80) return false;
     // One walking wave a workgroup has its CU's cache bandwidth to itself, two
     // share it but hand over in LDS what one would through memory, which pays
     // where walks are short and the K rows many: on
@@ -821,8 +829,8 @@ __global__ void k_wave_clear(v4u *p, unsigned n)
 }  // namespace
 
 // Allocates the packed sweeps' arrays; leaves c->ws null (the caller then uses
-// the natural-layout sweeps) when their offsets exceed 31 bits or the
-// memory is not there.
+// the natural-layout sweeps) on tall columns, when their offsets exceed 31 bits or
+// the memory is not there.
 int cad_wave_alloc(cad_ctx *c)
 {
     if (c->ws || c->ws_off) return CAD_OK;

@@ -194,3 +194,38 @@ def test_packed_sweeps_bitexact_with_oracle(pkg, shape):
     y = rs.standard_normal((ni, nj, nk))
     print(f"packed sweeps {shape}", flush=True)
     _milu_check(pkg, mat, indc, prm, "SWEEP_PIPELINED", [y, mat["BB"], y])
+
+
+@pytest.mark.parametrize("shape", [(2, 2, 200), (3, 3, 400)])
+def test_default_schedule_on_a_tall_column(pkg, shape):
+    """A column much taller than wide is a chain of tiles with next to no walk, on
+    which the packed sweeps take 1.4 times the 64-line tiles' time: the default
+    schedule takes the latter there, and equals the fixed tile shapes bit for bit.
+    (The bar of 1.15 lies between; the runs of one schedule differ by 1 %.)"""
+    ni, nj, nk = (n + 2 for n in shape)
+    indc = np.full((ni, nj, nk), -1, np.int32, order="F")
+    indc[1:-1, 1:-1, 1:-1] = 0
+    on = indc == 0
+    mat = {k: np.zeros((ni, nj, nk), order="F") for k in pkg.capi.MATRIX}
+    for a, (lo, up) in enumerate((("ALI", "AUI"), ("ALJ", "AUJ"), ("ALK", "AUK"))):
+        mat[lo][...] = np.where(on & np.roll(on, 1, axis=a), -1.0, 0.0)
+        mat[up][...] = np.where(on & np.roll(on, -1, axis=a), -1.0, 0.0)
+    mat["AD"][...] = 6.5
+    mat["BB"][...] = np.random.default_rng(5).standard_normal((ni, nj, nk))
+    lay = pkg.layout.from_text(pkg.configs.dam_break(*shape, col_x=0.01, col_z=0.01).deck)
+    ms, out = {}, {}
+    with pkg.capi.Context(ni, nj, nk, lay.numb) as c:
+        c.upload_static(lay.static_arrays())
+        c.upload_state(lay.raw_state())
+        c.set_params(cgpara=0.95, icgtyp=1, cgepsa=1e-15, cgepsr=1e-10, cgdiv=1e30, icgmax=500)
+        c.upload_matrix(mat, indc)
+        for name in ("SWEEP_PIPELINED", "SWEEP_PIPELINED_8X8", "SWEEP_PIPELINED_16X4"):
+            print(f"tall column {shape} {name}", flush=True)
+            c.set_sweep_schedule(getattr(pkg.capi, name))
+            c.milu_factor()
+            out[name] = c.milu_apply(mat["BB"])
+            c.time_minv(5)
+            ms[name] = sorted(c.time_minv(20) for _ in range(5))[2]
+    print(ms, flush=True)
+    assert all(np.array_equal(o, out["SWEEP_PIPELINED"]) for o in out.values())
+    assert ms["SWEEP_PIPELINED"] <= 1.15 * min(ms.values()), ms
