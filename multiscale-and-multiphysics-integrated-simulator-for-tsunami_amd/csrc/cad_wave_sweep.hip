@@ -774,11 +774,18 @@ bool wave_geometry(const Dims &d, cad_wsweep *ws, WSizes *z)
     if (d.nk - 2 >= 5 * std::max(d.ni - 2, d.nj - 2) + 80) return false;
     // One walking wave a workgroup has its CU's cache bandwidth to itself, two
     // share it but hand over in LDS what one would through memory, which pays
-    // where walks are short and the K rows many: on
-    // dam breaks (I x J x K) two against one measured 25 / 22 us on 30x16x16, 43 / 48 on
-    // 64x16x48, 68 / 68 on 64x64x48, 87 / 83 on 128x48x64, 91 / 88 on 512x16x64,
-    // 133 / 127 on 250x70x90, 149 / 133 on 512x100x64, 414 / 305 on 512x256x128.
-    const int nw = ws->nw = d.ni * d.nj < 4096 && d.nk >= 32 ? 2 : 1;
+    // where the K rows are many against the walk and the J tiles.  M^-1 of two / of
+    // one in us on tanks filled to 0.7 of their height, I x J x K, inside the line:
+    // 43 / 48 on 24x8x40, 34 / 37 on 16x16x32, 42 / 45 on 64x16x32, 63 / 70 on
+    // 30x16x64, 72 / 77 on 32x32x64, 120 / 130 on 20x20x128, 76 / 81 on 100x12x64, 68 / 69
+    // on 160x10x40, 61 / 60 on 64x16x48 (52 / 53 with water on a third of it), 89 / 90 on
+    // 100x30x64, 57 / 60 on 45x25x40, 48 / 47 on 48x12x36, 124 / 121 on 128x24x96.  Outside it: fewer K rows, 28 / 25 on
+    // 30x16x16, 43 / 40 on 64x16x24, 37 / 35 on 30x10x28; longer walks, 99 / 96 on
+    // 300x8x48; more J tiles, 186 / 152 on 2x300x50, 76 / 73 on 20x60x48, 72 / 70 on 36x36x48,
+    // 99 / 93 on 62x60x62; beyond 4096 cells of a plane 167 / 164 on 200x30x128, 89 / 82 on
+    // 64x64x48, 452 / 367 on 128x128x256.
+    const int ei = d.ni - 2, ej = d.nj - 2, ek = d.nk - 2;
+    const int nw = ws->nw = d.ni * d.nj < 4096 && ek >= 30 && 3 * ej <= 2 * ek && ei <= 4 * ek ? 2 : 1;
     WGeom &g = ws->g;
     g.ni = d.ni;
     g.nj = d.nj;

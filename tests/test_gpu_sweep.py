@@ -161,7 +161,7 @@ def test_milu_apply_bitexact_many_tiles(pkg, sched):
 
 
 @pytest.mark.parametrize("shape", [(4, 3, 3), (9, 16, 4), (14, 17, 9), (21, 2, 40), (37, 49, 5), (600, 11, 6),
-                                   (301, 21, 13)])
+                                   (301, 21, 13), (33, 30, 46), (20, 44, 67), (130, 9, 33)])
 def test_packed_sweeps_bitexact_with_oracle(pkg, shape):
     """The default schedule's packed sweeps at the edges of their tiles (16 x 4
     and 16 x 8 lines, stages of 8 steps, one and two walking waves a
