@@ -148,7 +148,8 @@ def test_unet_weight_gradients_by_segments_and_runs(pkg, box, nb):
     one 16-voxel segment on the coarsest level, x segments with a remainder
     (96 = 64 + 32 and 160 = 2 x 64 + 32 voxels on the middle level), row runs
     with a remainder, fewer and more units than blocks.  The bar is the one
-    above; the partial sums are added in a fixed order, so two calls give the
+    above, BF16's (test_unet_weight_gradients_equal_the_exact_sums compares without
+    rounding); the partial sums are added in a fixed order, so two calls give the
     same bits, apart from the output layer's 17 sums and what the loss's
     atomic sum moves: dy is given, so nothing."""
     import torch
@@ -179,3 +180,81 @@ def test_unet_weight_gradients_by_segments_and_runs(pkg, box, nb):
             print(f"{name} {'wb'[part]}: rel {rel:.3e}", flush=True)
             assert rel <= 1e-1, (name, part, rel)
             assert np.array_equal(a, g2[sl[name][part]]), (name, part)
+
+
+def _exact_case(pkg, box, nb, seed):
+    """Parameters, input and output gradient whose activations and gradients are
+    all short binary fractions: an output channel takes one input channel, or one of
+    each half, shifted by up to a voxel along x (weight 1, no bias), the input is 0 or 1,
+    the output gradient a sparse -1, 0 or 1.  Poolings divide by 8, so every value has
+    at most 8 significant bits (BF16 rounds nothing; checked here) and the weight
+    gradients' FP32 sums are exact."""
+    import torch
+    nx, ny, nz = box
+    rng = np.random.default_rng(seed)
+    U = pkg.unet
+    sl = U.layer_slices()
+    p = np.zeros(U.param_count(), np.float32)
+    for name in U.NAMES:
+        w, _, (ci, co) = sl[name]
+        k = np.zeros((27, ci, co), np.float32)
+        if ci > co:
+            chan = np.stack([rng.permutation(co), co + rng.permutation(co)])
+        else:
+            chan = np.concatenate([rng.permutation(ci) for _ in range(co // ci)])[None]
+        for c in chan:
+            k[rng.integers(12, 15, co), c, np.arange(co)] = 1.0
+        p[w] = k.ravel()
+    p[sl["out"][0]] = rng.choice([-1.0, 1.0], 16)
+    x = torch.from_numpy((rng.random((nb, 8, nz, ny, nx)) < 0.2).astype(np.float32))
+    xp = torch.zeros((nb, nz + 2, ny + 2, nx + 2, 8), dtype=torch.bfloat16)
+    xp[:, 1:-1, 1:-1, 1:-1, :] = x.permute(0, 2, 3, 4, 1)
+    dy = torch.from_numpy((rng.choice([-1.0, 1.0], (nb, nz, ny, nx)) * (rng.random((nb, nz, ny, nx)) < 0.05)).astype(np.float32))
+    prm = unet_ref.forward(U, p, x)
+    for v in prm.values():
+        v[0].requires_grad_(True)
+        v[1].requires_grad_(True)
+    seen = []
+
+    def keep(t):
+        t.retain_grad()
+        seen.append(t)
+        return t
+
+    relu, pool, up = torch.relu, torch.nn.functional.avg_pool3d, torch.nn.functional.interpolate
+    try:
+        torch.relu = lambda h: keep(relu(h))
+        torch.nn.functional.avg_pool3d = lambda *a, **k: keep(pool(*a, **k))
+        torch.nn.functional.interpolate = lambda *a, **k: keep(up(*a, **k))
+        y = unet_ref.run(prm, x)
+    finally:
+        torch.relu, torch.nn.functional.avg_pool3d, torch.nn.functional.interpolate = relu, pool, up
+    (y * dy).sum().backward()
+    for t in seen:
+        for v in (t.detach(), t.grad):
+            assert torch.equal(v.bfloat16().float(), v)
+    return p, xp, dy, unet_ref.grad_vector(U, prm, U.param_count())
+
+
+@pytest.mark.parametrize("box,nb", [((64, 4, 4), 1), ((192, 12, 20), 3), ((320, 36, 4), 1), ((128, 8, 12), 2)])
+def test_unet_weight_gradients_equal_the_exact_sums(pkg, box, nb):
+    """Weight and bias gradients of every tap and channel, where no rounding takes
+    part, equal the reference's: one voxel lost or taken twice at the edge of a
+    segment, a run or a plane changes a sum by at least 2^-12.  (Between the BF16
+    network and the FP32 one a layer's gradients differ by up to 0.1.)"""
+    U = pkg.unet
+    nx, ny, nz = box
+    p, xp, dy, want = _exact_case(pkg, box, nb, 3)
+    with U.UNet(nx, ny, nz, nb, train=True) as net:
+        import torch
+        net.set_params(p)
+        net.set_input(xp.cuda())
+        y = torch.empty(nb * nz * ny * nx, dtype=torch.float32, device="cuda")
+        net.forward(y)
+        g = net.gradients_dy(dy.reshape(-1).cuda())
+    sl = U.layer_slices()
+    for name in U.NAMES + ("out",):
+        for part in (0, 1):
+            a, b = g[sl[name][part]], want[sl[name][part]]
+            print(f"{name} {'wb'[part]}: {np.count_nonzero(b)} of {b.size} not 0, {np.count_nonzero(a != b)} differ", flush=True)
+            assert np.array_equal(a, b), (name, part, np.abs(a - b).max())
