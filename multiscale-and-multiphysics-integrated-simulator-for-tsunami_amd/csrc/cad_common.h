@@ -134,8 +134,7 @@ constexpr int CAD_REC = 8;        // first double of the solves' records in host
 // One level of the multigrid (cad_mg.hip): a grid with one ghost layer, its
 // 7-point rows (inactive rows AD = 1, no couplings), the level's unknowns and
 // right-hand side, and the row activity, stored colour by colour in lines of
-// ld cells; level 0 of the FP32 hierarchy also holds its rows and activity in
-// the grid's natural order (nad .. nauk, nact; null elsewhere).
+// ld cells.
 constexpr int CAD_MG_MAX = 12;
 template <typename V>
 struct MgLevelT {

@@ -51,8 +51,8 @@
 // 64x16x48 and 382 on 512x256x128, with two 46 and 368, with polls of one stage
 // and the J halo whole in its own entries 43 and 312.  M^-1 on water
 // of the workloads, against the 64-line tiles of cad_sweep.hip (whose step was 240
-// ns, waiting for its mailbox accesses): buildings 512x256x128 661 -> 312 us, run-up
-// 512x32x96 330 -> 155, 250x70x90 267 -> 129, dam break 64x16x48 61 -> 43.  Those
+// ns, waiting for its mailbox accesses): buildings 512x256x128 661 -> 313 us, run-up
+// 512x32x96 330 -> 157, 250x70x90 267 -> 130, dam break 64x16x48 61 -> 43.  Those
 // tiles stay for the factorisation, for the fixed tile shapes, on tall columns, and
 // where these arrays do not fit.
 #include "cad_common.h"
